@@ -31,19 +31,32 @@ MKD_DEV float gated_sigmoid(float g, float z) {
 // One gated activation value from the gate and up projections (fp32, bias
 // already added).  Qwen rounding: g, u -> bf16, silu(g) -> bf16, product;
 // otherwise clamps, then act(g) * u with act (kAct*) = silu, swish(alpha),
-// GELU (erf) or GELU's tanh approximation.
-MKD_DEV float swiglu_value(const GemmArgs& a, float gv, float uv) {
-  if (a.round_qwen) {
+// GELU (erf) or GELU's tanh approximation.  The kind is uniform over a launch.
+enum GatedKind { kGatedQwen, kGatedSigmoid, kGatedGelu };
+MKD_DEV int gated_kind(const GemmArgs& a) {
+  if (a.round_qwen) return kGatedQwen;
+  return a.act == kActGelu || a.act == kActGeluTanh ? kGatedGelu : kGatedSigmoid;
+}
+template <int KIND>
+MKD_DEV float gated_value(const GemmArgs& a, float gv, float uv) {
+  if (KIND == kGatedQwen) {
     const float g = rbf(gv), u = rbf(uv);
     return rbf(gated_sigmoid(g, g)) * u;
   }
   const float g = fmaxf(fminf(gv, a.gate_hi), a.gate_lo);
   const float u = fmaxf(fminf(uv, a.up_hi), a.up_lo);
-  if (a.act == kActGelu) return 0.5f * g * (1.0f + erff(g * 0.70710678118654752f)) * u;
-  if (a.act == kActGeluTanh)
+  if (KIND == kGatedGelu) {
+    if (a.act == kActGelu) return 0.5f * g * (1.0f + erff(g * 0.70710678118654752f)) * u;
     return 0.5f * g * (1.0f + tanhf(0.79788456080286536f * (g + 0.044715f * g * g * g))) * u;
+  }
   const float z = a.act == kActSwish ? a.alpha * g : g;
   return gated_sigmoid(g, z) * u;
+}
+MKD_DEV float swiglu_value(const GemmArgs& a, float gv, float uv) {
+  const int kind = gated_kind(a);
+  if (kind == kGatedQwen) return gated_value<kGatedQwen>(a, gv, uv);
+  if (kind == kGatedGelu) return gated_value<kGatedGelu>(a, gv, uv);
+  return gated_value<kGatedSigmoid>(a, gv, uv);
 }
 
 template <int RB, int TN, int EPI, bool COH = false>

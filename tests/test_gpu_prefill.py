@@ -89,3 +89,24 @@ def test_moe_prefill_rejects_unsupported(mk, dev):
     with pytest.raises(NotImplementedError):
         mk.moe_prefill(x, gu8, gu8, torch.zeros(4, 2, device=dev),
                        torch.zeros(4, 1, dtype=torch.int32, device=dev))
+
+
+# Group sizes at the edges of the token tiles (128) and of the inner loops (32, 64,
+# 96 and 128 tokens), and k steps (H / 32, I / 32) that leave the four-step loop
+# after any step.  Same tolerance as above: bf16 h and fp32 sums over K <= 416.
+@pytest.mark.parametrize("H,I", [(32, 32), (64, 96), (96, 160), (128, 224), (288, 64), (416, 128)])
+def test_moe_prefill_group_and_k_edges(mk, dev, H, I):
+    from nki_moe_megakernel_amd.common_types import ExpertAffinityScaleMode
+    counts = [0, 1, 31, 32, 33, 63, 64, 65, 95, 96, 97, 127, 128, 129, 160, 257, 0]
+    print(f"moe_prefill group edges H={H} I={I}", flush=True)
+    E, T = len(counts), sum(counts)
+    x, gu, dn, _, _, _, _ = _case(T, E, 1, H, I, False, seed=H + I)
+    g = torch.Generator().manual_seed(I)
+    idx = torch.repeat_interleave(torch.arange(E), torch.tensor(counts))[torch.randperm(T, generator=g)]
+    idx = idx.to(torch.int32).reshape(T, 1)
+    aff = torch.zeros(T, E).scatter_(1, idx.long(), torch.rand(T, 1, generator=g) + 0.5)
+    out = mk.moe_prefill(x.to(dev), gu.to(dev), dn.to(dev), aff.to(dev), idx.to(dev),
+                         expert_affinities_scaling_mode=ExpertAffinityScaleMode.POST_SCALE)
+    torch.cuda.synchronize()
+    y_ref = ref.moe_tkg(x, gu, dn, aff, idx.long(), None, None, "post", "silu")
+    assert max_abs_rel(out, y_ref) < TOL
