@@ -1505,8 +1505,10 @@ static hipError_t launch_tpw(const AttnArgs& a, int rope_mode, hipStream_t s) {
     if (hipError_t e = hipGetLastError()) return e;
   }
   const int chunk = a.chunk;
+  if (chunk >= 256 && attn_stream_ok(a)) return attn_stream_launch(a, s);
   if (chunk == 64) return launch_attn<D, GQA, 1>(a, rope_mode, s);
   if (chunk == 128) return launch_attn<D, GQA, 2>(a, rope_mode, s);
+  // (block lengths that are no multiple of 16, unaligned caches)
   if (chunk == 256) return launch_attn<D, GQA, 4>(a, rope_mode, s);
   return hipErrorInvalidValue;
 }

@@ -931,7 +931,7 @@ static int attention_core(const mkd_attention_args* p, AttnWs& w, const int* pos
   a.part_o = w.po; a.part_ml = w.pml;
   // large grids prepare the q / k / v heads once per (sequence, kv head) in a
   // launch of their own; small ones inside every attention block
-  a.prep = (NT > 1 || (long long)w.n_chunks * p->nkv * rows > 1024) ? w.prep : nullptr;
+  a.prep = (NT > 1 || w.chunk >= 256 || (long long)w.n_chunks * p->nkv * rows > 1024) ? w.prep : nullptr;
   a.attn_out = w.attn;
   a.update_cache = p->update_cache;
   a.write_pos = p->kv_cache_update_idx;
@@ -969,6 +969,10 @@ static int attention_core(const mkd_attention_args* p, AttnWs& w, const int* pos
   // the caller left its router to the joined launch
   MKD_REQUIRE(!(join && join->rw), MKD_ERR_UNSUPPORTED,
               "attention: the joined launch with its router stage does not fit this layer");
+  if ((a.chunk >= 256 || a.kv_fp8) && attn_stream_ok(a)) {
+    a.chunk = attn_stream_chunk(a);
+    a.n_chunks = (a.S_max + NT + a.chunk - 1) / a.chunk;
+  }
   if (kvfmt) {
     MKD_REQUIRE(!prefill && a.window == 0, MKD_ERR_UNSUPPORTED,
                 "attention: fp8 / transposed-K caches are served by the operator path only");

@@ -328,6 +328,12 @@ hipError_t attn_combine_launch(const AttnArgs& a, hipStream_t s);
 int attn_chunk_for(int B, int nkv, int S_max);   // positions per attention block (64/128/256)
 // q / k / v head preparation of every (row, kv head) into a.prep (required)
 hipError_t attn_prep_launch(const AttnArgs& a, int rope_mode, hipStream_t s);
+// attn_stream.hip: the chunk kernel of grids that fill the chip (chunk >= 256) and
+// of FP8 caches; whether it takes these arguments, and its chunk
+bool attn_stream_ok(const AttnArgs& a);
+int attn_stream_chunk(const AttnArgs& a);
+hipError_t attn_stream_launch(const AttnArgs& a, hipStream_t s);
+
 // Option-path attention over fp8 / transposed-K caches (attn_kvfmt.hip): the
 // head preparation, then split-K chunk partials in the layout attn_combine
 // merges; the new rows are stored afterwards by attn_kvfmt_store_launch, after

@@ -1,0 +1,99 @@
+"""The streaming decode attention (grids of >= 1024 chunk blocks, FP8 row caches) against the
+oracle, at the edges of its steps (32 positions), chunks (64 .. 512) and cache blocks, and the
+block lengths it leaves to the general kernels.
+
+Tolerance: max-abs-rel 2e-2, the bf16 bound of the other attention tests (probabilities rounded to
+bf16, or hi + lo for FP8, and a bf16 output).  The same logical cache through block lengths 16 / 32 /
+64 (streaming) and 24 (general kernels) differs only by the two kernels' summation orders and their
+bf16 roundings of the probabilities: held to 1e-2.
+"""
+import pytest
+import torch
+
+from conftest import max_abs_rel
+from oracle import ref
+from test_gpu_kv_formats import _call, _rope_rows, bf
+
+pytestmark = pytest.mark.gpu
+
+
+def _run(mk, dev, fp8, blk, B, nq, nkv, d, NT, P, seed=3):
+    """The operator and the oracle on one case: (out, oracle out), both [B, nq, d, NT]."""
+    g = torch.Generator().manual_seed(seed + B + P)
+    H, gqa = 128, nq // nkv
+    S_max = P + NT + 5 if not blk else (P + NT + blk - 1) // blk * blk
+    S_ctx = S_max if blk else P + NT           # a block cache's mask covers its whole table
+    prior = S_ctx - NT
+    X = bf(torch.randn(B, NT, H, generator=g))
+    W = bf(0.05 * torch.randn(H, d * (nq + 2 * nkv), generator=g))
+    K = torch.randn(B, nkv, S_max, d, generator=g)
+    V = torch.randn(B, nkv, S_max, d, generator=g)
+    ks = vs = None
+    if fp8:
+        K, V = ref.kv_fp8_quant(K, 8.0), ref.kv_fp8_quant(V, 8.0)
+        ks = vs = torch.full((1, 1), 8.0)
+    else:
+        K, V = bf(K), bf(V)
+    # ragged lengths, single masked positions and a whole masked 64-position stretch
+    lens = torch.randint(max(P // 2, 0), P + 1, (B,), generator=g)
+    lens[0] = P
+    keep = (torch.arange(prior)[:, None] < lens[None, :])[:, :, None, None].expand(prior, B, nq, NT).clone()
+    keep &= torch.rand(prior, B, nq, NT, generator=g) < 0.9
+    keep[P // 2: P // 2 + 64] = False
+    mask = torch.cat([keep, torch.ones(NT, B, nq, NT, dtype=torch.bool)]).to(torch.uint8)
+    cos, sin = _rope_rows(B, NT, P, d)
+    upd = torch.full((B, 1), 0xFFFFFFFF, dtype=torch.int64)
+    scale = d ** -0.5 / (8.0 if fp8 else 1.0)
+    table = None
+    Kd, Vd = K, V
+    if blk:
+        nb = S_max // blk
+        table = torch.randperm(B * nb, generator=g).to(torch.int32).reshape(B, nb)
+        pool = [torch.empty(B * nb, blk, nkv, d, dtype=K.dtype) for _ in range(2)]
+        for t, p in ((K, pool[0]), (V, pool[1])):
+            p.view(torch.uint8)[table.reshape(-1).long()] = \
+                t.transpose(1, 2).reshape(B * nb, blk, nkv, d).contiguous().view(torch.uint8)
+        Kd, Vd = pool
+    Kg, Vg = Kd.contiguous().to(dev), Vd.contiguous().to(dev)
+    out, _, _ = _call(mk, dev, X, W, None, None, None, cos, sin, Kg, Vg, mask, None, upd, table, False,
+                      ks, vs, scale)
+    torch.cuda.synchronize()
+    attn = torch.zeros(B * NT, nq * d)
+    for h in range(nkv):
+        cols = torch.cat([torch.arange(h * gqa * d, (h + 1) * gqa * d), nq * d + h * d + torch.arange(d),
+                          (nq + nkv) * d + h * d + torch.arange(d)])
+        o, _, _ = ref.attention_block_tkg(
+            X.float(), W.float()[:, cols], None, 1e-6, None, None, None, 1e-6, cos, sin, K[:, h].clone(),
+            V[:, h].clone(), mask[:, :, h * gqa:(h + 1) * gqa].float(), None, False, upd, None, None,
+            softmax_scale=scale, k_scale=8.0 if fp8 else None, v_scale=8.0 if fp8 else None)
+        attn[:, h * gqa * d:(h + 1) * gqa * d] = o
+    return out, attn.reshape(B, NT, nq, d).permute(0, 2, 3, 1)
+
+
+@pytest.mark.parametrize("blk,B,nq,nkv,d,NT,P", [
+    (0, 1, 8, 1, 128, 1, 0), (0, 1, 8, 1, 128, 1, 1), (0, 2, 4, 2, 64, 1, 31), (0, 1, 16, 1, 128, 1, 32),
+    (16, 2, 2, 2, 64, 1, 63), (64, 1, 8, 1, 128, 3, 64), (0, 3, 8, 2, 64, 8, 129), (32, 4, 8, 4, 128, 1, 500),
+    (24, 2, 8, 2, 128, 1, 100), (64, 64, 16, 8, 64, 1, 640), (0, 64, 16, 16, 64, 2, 300)])
+def test_fp8_stream_matches_oracle(mk, dev, blk, B, nq, nkv, d, NT, P):
+    print(f"fp8 stream blk={blk} B={B} nq={nq} nkv={nkv} d={d} NT={NT} P={P}", flush=True)
+    out, want = _run(mk, dev, True, blk, B, nq, nkv, d, NT, P)
+    assert max_abs_rel(out, want) < 2e-2
+
+
+# >= 1024 blocks of 256 positions: the streaming kernel; from 2048 blocks of 512: its larger chunk
+@pytest.mark.parametrize("blk,B,nq,nkv,d,NT,P", [
+    (0, 64, 16, 16, 64, 1, 255), (16, 64, 32, 16, 64, 1, 300), (64, 64, 16, 8, 128, 1, 511),
+    (0, 64, 8, 8, 128, 2, 257), (32, 128, 16, 16, 64, 1, 513)])
+def test_bf16_stream_matches_oracle(mk, dev, blk, B, nq, nkv, d, NT, P):
+    print(f"bf16 stream blk={blk} B={B} nq={nq} nkv={nkv} d={d} NT={NT} P={P}", flush=True)
+    out, want = _run(mk, dev, False, blk, B, nq, nkv, d, NT, P)
+    assert max_abs_rel(out, want) < 2e-2
+
+
+@pytest.mark.parametrize("fp8", [False, True])
+def test_stream_equals_general_path(mk, dev, fp8):
+    """The same logical cache (192 positions per table) in blocks of 16 / 32 / 64 rows and, through the
+    general kernels, of 24."""
+    outs = [_run(mk, dev, fp8, blk, 128, 16, 8, 64, 1, 191)[0] for blk in (16, 32, 64, 24)]
+    for o in outs[:3]:
+        assert max_abs_rel(o, outs[3].float()) < 1e-2
