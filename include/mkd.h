@@ -332,6 +332,33 @@ int mkd_pack_fp8_weights(const void* src, void* dst, int G, int N, int K, void* 
 size_t mkd_attention_workspace_bytes_tkg(int B, int s_tkg, int H, int nq, int nkv, int d, int S_max);
 int mkd_attention_block_tkg(const mkd_attention_args* args, void* workspace,
                             size_t workspace_bytes, void* stream);
+/* The small operands of mkd_attention_block_tkg from the reference operator's
+ * forms (attention_block_tkg.py:101-103, :115-121), in one launch:
+ *  - cos / sin [d/2, B, s_tkg] (fp32 or bf16, any strides in elements, each with
+ *    its own) -> cos_out / sin_out [B * s_tkg, d] fp32, halves duplicated; NULL
+ *    cos: none;
+ *  - n_prior_out [B] filled with n_prior;
+ *  - update_idx [B] int64 (stride in elements) -> write_pos_out int32, -1 (skip)
+ *    for UINT32_MAX, negative and larger than INT32_MAX values; NULL: none;
+ *  - table [table_rows, table_cols] int64 (strides in elements) -> table_out
+ *    int32, -1 outside [0, num_blocks); NULL: none. */
+typedef struct {
+  const void *cos, *sin;
+  int rope_dtype;              /* MKD_DT_* of both */
+  long long cos_stride[3], sin_stride[3];
+  float *cos_out, *sin_out;
+  int B, s_tkg, d;
+  int n_prior;
+  int* n_prior_out;
+  const long long* update_idx;
+  long long update_stride;
+  int* write_pos_out;
+  const long long* table;
+  long long table_stride[2];
+  int table_rows, table_cols, num_blocks;
+  int* table_out;
+} mkd_attention_operands;
+int mkd_attention_prepare_operands(const mkd_attention_operands* ops, void* stream);
 
 /* ---------------------------------------------------------------------------
  * Multi-layer Qwen3-MoE decode step -- replaces the megakernel

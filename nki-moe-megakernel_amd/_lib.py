@@ -77,6 +77,16 @@ class AttentionArgs(C.Structure):
     ]
 
 
+class AttentionOperands(C.Structure):
+    _fields_ = [
+        ("cos", vp), ("sin", vp), ("rope_dtype", i32), ("cos_stride", i64 * 3), ("sin_stride", i64 * 3),
+        ("cos_out", vp), ("sin_out", vp), ("B", i32), ("s_tkg", i32), ("d", i32), ("n_prior", i32),
+        ("n_prior_out", vp), ("update_idx", vp), ("update_stride", i64), ("write_pos_out", vp),
+        ("table", vp), ("table_stride", i64 * 2), ("table_rows", i32), ("table_cols", i32),
+        ("num_blocks", i32), ("table_out", vp),
+    ]
+
+
 KV_FP8 = 1            # MKD_KV_FP8
 KV_K_TRANSPOSED = 2   # MKD_KV_K_TRANSPOSED
 
@@ -120,6 +130,7 @@ _SIGS = {
     "mkd_attention_workspace_bytes": (sz, [i32, i32, i32, i32, i32, i32]),
     "mkd_attention_workspace_bytes_tkg": (sz, [i32, i32, i32, i32, i32, i32, i32]),
     "mkd_attention_block_tkg": (i32, [C.POINTER(AttentionArgs), vp, sz, vp]),
+    "mkd_attention_prepare_operands": (i32, [C.POINTER(AttentionOperands), vp]),
     "mkd_packed_fp8_bytes": (sz, [i32, i32, i32]),
     "mkd_pack_fp8_weights": (i32, [vp, vp, i32, i32, i32, vp]),
     "mkd_qwen3_workspace_bytes": (sz, [C.POINTER(Qwen3Model), i32]),

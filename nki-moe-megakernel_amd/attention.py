@@ -10,8 +10,6 @@ from . import _lib as L
 from . import packing
 from .common_types import QuantizationType
 
-U32_MAX = 0xFFFFFFFF
-
 
 def attention_block_tkg(
     X: torch.Tensor, X_hidden_dim_actual: Optional[int],
@@ -212,24 +210,48 @@ def attention_block_tkg(
             if rmsnorm_QK_post_rope_W_Q is not None else torch.ones(d, dtype=torch.bfloat16, device=dev)
         kp = rmsnorm_QK_post_rope_W_K.reshape(-1).to(torch.bfloat16).contiguous() \
             if rmsnorm_QK_post_rope_W_K is not None else torch.ones(d, dtype=torch.bfloat16, device=dev)
-    cos_f = sin_f = None
+    # [S_ctx, B, nq, S_tkg]; the kernels test bytes against zero (with S_tkg = 1 they read [S_ctx, B, nq])
+    if attention_mask.dtype in (torch.uint8, torch.bool):
+        mask_u8 = attention_mask.contiguous()
+    else:
+        mask_u8 = (attention_mask != 0).to(torch.uint8).contiguous()
+    # RoPE rows, prior lengths, write positions and block table in the kernels' forms
+    # (mkd_attention_prepare_operands): [cos | sin | n_prior | wpos | table] in one buffer.  int32
+    # positions and tables go to the kernels as they are: values that name no row are skipped there.
+    if cos is not None and (cos.dtype != sin.dtype or cos.dtype not in (torch.float32, torch.bfloat16)):
+        cos, sin = cos.float(), sin.float()
+    idx = kv_cache_update_idx.reshape(-1) if update_cache else None
+    if idx is not None and idx.dtype != torch.int32:
+        idx = idx.to(torch.int64)
+    table = active_blocks_table
+    if block and table.dtype != torch.int32:
+        table = table.to(torch.int64)
+    L.require_gpu(cos, sin, idx, table)
+    n_rope = B * S_tkg * d if cos is not None else 0
+    conv_idx = idx is not None and idx.dtype == torch.int64
+    conv_table = block and table.dtype == torch.int64
+    small = torch.empty(2 * n_rope + 2 * B + (table.numel() if conv_table else 0), dtype=torch.int32, device=dev)
+    base = small.data_ptr()
+    cos_p, sin_p, n_prior_p = base, base + 4 * n_rope, base + 8 * n_rope
+    wpos_p, table_p = n_prior_p + 4 * B, n_prior_p + 8 * B
+    ops = L.AttentionOperands(B=B, s_tkg=S_tkg, d=d, n_prior=S_ctx - S_tkg, n_prior_out=n_prior_p)
     if cos is not None:
-        # [d/2, B, S_tkg] -> [B * S_tkg, d] with the halves duplicated (row b * S_tkg + s)
-        cos_f = torch.cat([cos, cos], 0).permute(1, 2, 0).reshape(B * S_tkg, d).float().contiguous()
-        sin_f = torch.cat([sin, sin], 0).permute(1, 2, 0).reshape(B * S_tkg, d).float().contiguous()
-    # [S_ctx, B, nq, S_tkg] 0/1 (with S_tkg = 1 the kernel reads it as [S_ctx, B, nq])
-    mask_u8 = (attention_mask != 0).to(torch.uint8).contiguous()
-    n_prior = torch.full((B,), S_ctx - S_tkg, dtype=torch.int32, device=dev)
-    wpos = None
-    if update_cache:
-        idx = kv_cache_update_idx.reshape(-1).to(torch.int64)
-        wpos = torch.where((idx == U32_MAX) | (idx < 0) | (idx > 0x7FFFFFFF),
-                           torch.full_like(idx, -1), idx).to(torch.int32).contiguous()
-    table = None
-    if block:
-        t64 = active_blocks_table.to(torch.int64)
-        table = torch.where((t64 < 0) | (t64 >= num_blocks), torch.full_like(t64, -1), t64) \
-            .to(torch.int32).contiguous()
+        ops.cos, ops.sin, ops.cos_out, ops.sin_out = cos.data_ptr(), sin.data_ptr(), cos_p, sin_p
+        ops.rope_dtype = L.DT_F32 if cos.dtype == torch.float32 else L.DT_BF16
+        ops.cos_stride[:] = cos.stride()
+        ops.sin_stride[:] = sin.stride()
+    if conv_idx:
+        ops.update_idx, ops.update_stride, ops.write_pos_out = idx.data_ptr(), idx.stride(0), wpos_p
+    elif idx is not None:
+        idx = idx.contiguous()
+        wpos_p = idx.data_ptr()
+    if conv_table:
+        ops.table, ops.table_out, ops.num_blocks = table.data_ptr(), table_p, num_blocks
+        ops.table_stride[:] = table.stride()
+        ops.table_rows, ops.table_cols = table.shape
+    elif block:
+        table = table.contiguous()
+        table_p = table.data_ptr()
     sink_f = sink.reshape(-1).float().contiguous() if sink is not None else None
     ks = vs = None
     if kv_quant:   # element 0 of each scale, as fp32 on the device (no host round trip)
@@ -243,13 +265,13 @@ def attention_block_tkg(
         X=x.data_ptr(), rmsnorm_gamma=L.ptr(gamma),
         rmsnorm_eps=float(rmsnorm_X_eps if rmsnorm_X_eps is not None else 1e-3), rmsnorm_order=0,
         w_qkv_packed=wqkv.data_ptr(), bias_qkv=L.ptr(bqkv), q_norm=L.ptr(qn), k_norm=L.ptr(kn),
-        qk_eps=float(rmsnorm_QK_pre_rope_eps), cos=L.ptr(cos_f), sin=L.ptr(sin_f),
-        k_cache=K_cache.data_ptr(), v_cache=V_cache.data_ptr(), n_prior=n_prior.data_ptr(),
+        qk_eps=float(rmsnorm_QK_pre_rope_eps), cos=cos_p if cos is not None else None, sin=sin_p if cos is not None else None,
+        k_cache=K_cache.data_ptr(), v_cache=V_cache.data_ptr(), n_prior=n_prior_p,
         mask=mask_u8.data_ptr(), mask_s_ctx=S_ctx, sink=L.ptr(sink_f), softmax_scale=scale,
-        update_cache=int(bool(update_cache)), kv_cache_update_idx=L.ptr(wpos),
+        update_cache=int(bool(update_cache)), kv_cache_update_idx=wpos_p if idx is not None else None,
         w_out_packed=L.ptr(wout), bias_out=L.ptr(bout), residual=None, out=out.data_ptr(),
         B=B, H=H, H_out=H_out, nq=nq, nkv=nkv, d=d, S_max=S_max, round_qwen=0,
-        active_blocks_table=L.ptr(table), blocks_per_seq=table.shape[1] if block else 0,
+        active_blocks_table=table_p if block else None, blocks_per_seq=table.shape[1] if block else 0,
         block_len=blk_len if block else 0, num_blocks=num_blocks if block else 0, s_tkg=S_tkg,
         q_norm_post=L.ptr(qp), k_norm_post=L.ptr(kp),
         qk_post_eps=float(rmsnorm_QK_post_rope_eps) if rmsnorm_QK_post_rope_enabled else 0.0,
@@ -258,9 +280,11 @@ def attention_block_tkg(
         quant_qkv=1 if q_static else 0, quant_out=1 if o_static else 0,
         w_scale_qkv=L.ptr(wsq), in_scale_qkv=L.ptr(isq), w_scale_out=L.ptr(wso), in_scale_out=L.ptr(iso))
     lib = L.load()
-    ws = torch.zeros(max(lib.mkd_attention_workspace_bytes_tkg(B, S_tkg, H, nq, nkv, d, S_max), 256),
+    ws = torch.empty(max(lib.mkd_attention_workspace_bytes_tkg(B, S_tkg, H, nq, nkv, d, S_max), 256),
                      dtype=torch.uint8, device=dev)
-    rc = lib.mkd_attention_block_tkg(args, ws.data_ptr(), ws.numel(), L.stream_ptr(dev))
+    stream = L.stream_ptr(dev)
+    L.check(lib.mkd_attention_prepare_operands(ops, stream), "attention_block_tkg")
+    rc = lib.mkd_attention_block_tkg(args, ws.data_ptr(), ws.numel(), stream)
     L.check(rc, "attention_block_tkg")
     if W_out is None:   # [B, q_heads, d_head, S_tkg]
         out = out.reshape(B, S_tkg, nq, d).permute(0, 2, 3, 1).contiguous()

@@ -1726,6 +1726,22 @@ int mkd_qwen3_prefill_layers(const mkd_qwen3_model* m, int seq, int T, void* hid
   return decode_layers(m, T, hidden, position_ids, cos, sin, workspace, workspace_bytes, stream, seq);
 }
 
+int mkd_attention_prepare_operands(const mkd_attention_operands* o, void* stream) {
+  if (int rc = stale_check("mkd_attention_prepare_operands")) return rc;
+  MKD_REQUIRE(o && o->n_prior_out, MKD_ERR_NULL, "attention operands: null pointer");
+  MKD_REQUIRE(o->B > 0 && o->s_tkg > 0 && o->d > 0 && o->d % 2 == 0 &&
+                  (long long)o->B * o->s_tkg * o->d < (1LL << 31) &&
+                  (o->rope_dtype == MKD_DT_F32 || o->rope_dtype == MKD_DT_BF16),
+              MKD_ERR_INVALID, "attention operands: bad shape");
+  MKD_REQUIRE(!o->cos || (o->sin && o->cos_out && o->sin_out), MKD_ERR_NULL, "attention operands: null RoPE table");
+  MKD_REQUIRE(!o->update_idx || o->write_pos_out, MKD_ERR_NULL, "attention operands: null write positions");
+  MKD_REQUIRE(!o->table || (o->table_out && o->table_rows > 0 && o->table_cols > 0 &&
+                            (long long)o->table_rows * o->table_cols < (1LL << 31)),
+              MKD_ERR_INVALID, "attention operands: bad block table");
+  MKD_TRY(attn_operands_launch(*o, static_cast<hipStream_t>(stream)), "attention operands");
+  return MKD_OK;
+}
+
 int mkd_embed(const int* token_ids, const void* table, void* out, int B, int H, int V,
               void* stream) {
   if (int rc = stale_check("mkd_embed")) return rc;

@@ -2,6 +2,8 @@
 #include "common.h"
 #include "mkd_internal.h"
 
+#include <algorithm>
+
 namespace mkd {
 
 __global__ void embed_kernel(const int* __restrict__ ids, const uint16_t* __restrict__ table,
@@ -13,6 +15,40 @@ __global__ void embed_kernel(const int* __restrict__ ids, const uint16_t* __rest
   // an out-of-vocabulary id yields a zero row instead of a read outside the table
   const u32x4_t z = {0, 0, 0, 0};
   st16(out + (long long)b * H + i, (id >= 0 && id < V) ? ld16(table + (long long)id * H + i) : z);
+}
+
+// The attention operator's small operands (mkd_attention_operands) in one launch: as
+// torch operations they were ~15 launches of a few microseconds each, which set the
+// operator's time at small batches (4 sequences x 2048 positions: 136 us a call, of
+// which ~35 us of attention kernels).  One thread per element of the largest.
+MKD_DEV float rope_at(const void* p, int dt, long long i) {
+  return dt == MKD_DT_F32 ? static_cast<const float*>(p)[i] : bf2f(static_cast<const uint16_t*>(p)[i]);
+}
+__global__ void __launch_bounds__(256) attn_operands_kernel(mkd_attention_operands o) {
+  const int i = blockIdx.x * 256 + threadIdx.x;
+  if (o.cos && i < o.B * o.s_tkg * o.d) {
+    const int row = i / o.d, e = i % o.d;
+    const int h = e < o.d / 2 ? e : e - o.d / 2, b = row / o.s_tkg, t = row % o.s_tkg;
+    o.cos_out[i] = rope_at(o.cos, o.rope_dtype, h * o.cos_stride[0] + b * o.cos_stride[1] + t * o.cos_stride[2]);
+    o.sin_out[i] = rope_at(o.sin, o.rope_dtype, h * o.sin_stride[0] + b * o.sin_stride[1] + t * o.sin_stride[2]);
+  }
+  if (i < o.B) {
+    o.n_prior_out[i] = o.n_prior;
+    if (o.update_idx) {
+      const long long v = o.update_idx[i * o.update_stride];
+      o.write_pos_out[i] = v < 0 || v > 0x7fffffffLL ? -1 : (int)v;   // (UINT32_MAX among them)
+    }
+  }
+  if (o.table && i < o.table_rows * o.table_cols) {
+    const long long v = o.table[(i / o.table_cols) * o.table_stride[0] + (i % o.table_cols) * o.table_stride[1]];
+    o.table_out[i] = v < 0 || v >= o.num_blocks ? -1 : (int)v;
+  }
+}
+hipError_t attn_operands_launch(const mkd_attention_operands& o, hipStream_t s) {
+  const long long n = std::max({o.cos ? (long long)o.B * o.s_tkg * o.d : 0LL, (long long)o.B,
+                                o.table ? (long long)o.table_rows * o.table_cols : 0LL});
+  hipLaunchKernelGGL(attn_operands_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, o);
+  return hipGetLastError();
 }
 
 // Stage 1: each block reduces a slice of one row to (max, first index).

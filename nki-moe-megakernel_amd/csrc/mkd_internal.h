@@ -4,6 +4,8 @@
 #include <hip/hip_ext.h>
 #include <stdint.h>
 
+#include "mkd.h"
+
 namespace mkd {
 
 enum Epi { EPI_F32 = 0, EPI_BF16 = 1, EPI_RESID_BF16 = 2, EPI_SWIGLU_BF16 = 3, EPI_SCALE_F32 = 4 };
@@ -549,6 +551,7 @@ hipError_t moe_finalize_launch(const float* ybuf, int T, int K, int H, const uin
                                uint16_t* out, float* out_f32, hipStream_t s);
 
 // misc.hip
+hipError_t attn_operands_launch(const mkd_attention_operands& o, hipStream_t s);
 hipError_t embed_launch(const int* ids, const uint16_t* table, uint16_t* out, int B, int H, int V,
                         hipStream_t s);
 hipError_t argmax_launch(const float* logits, int B, int V, int* out, float* scratch_val,

@@ -75,10 +75,16 @@ def router_topk(x: torch.Tensor, w: torch.Tensor, w_bias: Optional[torch.Tensor]
     if xt.dtype not in (torch.float32, torch.bfloat16):
         raise ValueError("x must be bfloat16 or float32")
     dev = x.device
-    logits = torch.empty(T, E, dtype=torch.float32, device=dev)
-    aff = torch.empty(T, E, dtype=torch.float32, device=dev)
-    idx = torch.empty(T, k, dtype=torch.int32, device=dev)
-    topk = torch.empty(T, k, dtype=torch.float32, device=dev)
+    # the kernels write the caller's tensors where their layout is the kernels' own (no copies after)
+    def direct(t, shape, dtype, wanted=True):
+        if (wanted and t.dtype == dtype and tuple(t.shape) == shape and t.is_contiguous()
+                and t.device == dev and t.data_ptr() % 16 == 0):
+            return t
+        return torch.empty(shape, dtype=dtype, device=dev)
+    logits = direct(router_logits, (T, E), torch.float32)
+    aff = direct(expert_affinities, (T, E), torch.float32)
+    idx = direct(expert_index, (T, k), torch.int32, not skip_store_expert_index)
+    topk = torch.empty(T, k, dtype=torch.float32, device=dev) if return_eager_affi else None
     mode = 0
     if act_fn == RouterActFnType.SIGMOID:
         mode |= L.ROUTER_SIGMOID
@@ -93,12 +99,15 @@ def router_topk(x: torch.Tensor, w: torch.Tensor, w_bias: Optional[torch.Tensor]
         t1 = min(T, t0 + 4096)
         rc = lib.mkd_router_topk(xt[t0:t1].data_ptr(), xdt, t1 - t0, H, wp.data_ptr(), E,
                                  L.ptr(bias), logits[t0:t1].data_ptr(), aff[t0:t1].data_ptr(),
-                                 idx[t0:t1].data_ptr(), topk[t0:t1].data_ptr(), k, mode,
+                                 idx[t0:t1].data_ptr(), topk[t0:t1].data_ptr() if topk is not None else None,
+                                 k, mode,
                                  ws.data_ptr(), ws.numel(), L.stream_ptr(dev))
         L.check(rc, "router_topk")
-    router_logits.copy_(logits)
-    expert_affinities.copy_(aff)
-    if not skip_store_expert_index:
+    if logits is not router_logits:
+        router_logits.copy_(logits)
+    if aff is not expert_affinities:
+        expert_affinities.copy_(aff)
+    if idx is not expert_index and not skip_store_expert_index:
         expert_index.copy_(idx)
     out = [router_logits, expert_index, expert_affinities]
     if return_eager_affi:

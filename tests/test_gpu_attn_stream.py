@@ -97,3 +97,70 @@ def test_stream_equals_general_path(mk, dev, fp8):
     outs = [_run(mk, dev, fp8, blk, 128, 16, 8, 64, 1, 191)[0] for blk in (16, 32, 64, 24)]
     for o in outs[:3]:
         assert max_abs_rel(o, outs[3].float()) < 1e-2
+
+
+@pytest.mark.parametrize("blk", [0, 16])
+@pytest.mark.parametrize("form", ["int64", "strided", "bf16 rope", "mask bool", "mask bf16"])
+def test_operand_forms_agree(mk, dev, blk, form):
+    """Write positions, block tables, masks and RoPE tables in the other dtypes and strides the operator
+    takes give bit for bit the result of their plain forms, out-of-range entries included."""
+    g = torch.Generator().manual_seed(9)
+    B, H, nq, nkv, d, S = 3, 256, 8, 2, 64, 48
+    X, W = bf(torch.randn(B, 1, H, generator=g)), bf(0.05 * torch.randn(H, d * (nq + 2 * nkv), generator=g))
+    shape = (B * 3, 16, nkv, d) if blk else (B, nkv, S, d)
+    K, V = bf(torch.randn(shape, generator=g)), bf(torch.randn(shape, generator=g))
+    cos, sin = [bf(t).float() for t in _rope_rows(B, 1, S - 1, d)]
+    mask = (torch.rand(S, B, nq, 1, generator=g) < 0.8).to(torch.uint8)
+    upd = torch.tensor([5, -1, 40], dtype=torch.int32)[:, None]
+    table = torch.arange(B * 3, dtype=torch.int32).reshape(B, 3) if blk else None
+    if blk:
+        table[1, 2], table[2, 0] = -7, B * 3 + 100           # no such blocks: rows read as zero
+
+    def call(cos, sin, mask, upd, table):
+        Kg, Vg = K.to(dev), V.to(dev)
+        from nki_moe_megakernel_amd.common_types import QuantizationType as QT
+        out, _, _ = mk.attention_block_tkg(
+            X.to(dev), None, False, 1e-6, None, W.to(dev), None, QT.NONE, None, None, False, 1e-6, None, None,
+            cos, sin, True, False, 1e-6, None, None, False, table, Kg, Vg, mask, None, True, upd, None, None,
+            QT.NONE, None, None, False, False)
+        return out, Kg, Vg
+    tb = table.to(dev) if blk else None
+    base = call(cos.to(dev), sin.to(dev), mask.to(dev), upd.to(dev), tb)
+    c, s, m, u = cos.to(dev), sin.to(dev), mask.to(dev), upd.to(dev)
+    if form == "int64":
+        u = torch.tensor([5, 0xFFFFFFFF, 40], device=dev)[:, None]
+        tb = tb.long() if blk else None
+        if blk:
+            tb[2, 0] = (1 << 33) + 1                          # its low 32 bits name a block
+    elif form == "strided":
+        c = torch.cat([c, c], 2)[:, :, :1]
+        s = s.permute(1, 2, 0).contiguous().permute(2, 0, 1)
+        u = torch.cat([u, u], 1).long()[:, 1:]
+        tb = torch.cat([tb, tb], 1).long()[:, 3:] if blk else None
+        m = torch.cat([m, m], 3)[..., :1]
+    elif form == "bf16 rope":
+        c, s = c.bfloat16(), s.bfloat16()
+    else:
+        m = m.to(torch.bool if form == "mask bool" else torch.bfloat16)
+    got = call(c, s, m, u, tb)
+    for a, b in zip(got, base):
+        assert torch.equal(a, b)
+
+
+def test_router_writes_callers_tensors(mk, dev):
+    """Outputs of the kernels' own layout are written in place; strided or otherwise typed ones get the
+    same values."""
+    g = torch.Generator().manual_seed(4)
+    T, H, E, k = 33, 256, 128, 8
+    x, w = torch.randn(T, H, generator=g).to(dev), bf(torch.randn(H, E, generator=g)).float().to(dev)
+
+    def call(lg, af, ix):
+        r = mk.router_topk(x, w, None, lg, af, ix, mk.RouterActFnType.SOFTMAX, k, 1, 0, True, True)
+        assert r[0] is lg and r[1] is ix and r[2] is af
+        return lg, af, ix
+    a = call(torch.empty(T, E, device=dev), torch.empty(T, E, device=dev),
+             torch.empty(T, k, dtype=torch.int32, device=dev))
+    b = call(torch.empty(E, T, device=dev).t(), torch.empty(T * E + 1, device=dev)[1:].reshape(T, E),
+             torch.empty(T, k, dtype=torch.int64, device=dev))
+    for p, q in zip(a, b):
+        assert torch.equal(p, q.to(p.dtype))
