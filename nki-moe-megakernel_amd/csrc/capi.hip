@@ -282,19 +282,6 @@ MoeWs carve_moe(Carver& c, int T, int H, int E, int I, int K) {
   return w;
 }
 
-__global__ void gather_slot_weights(const float* aff, const int* idx, int T, int E, int K,
-                                    float* slot_w) {
-  const int p = blockIdx.x * blockDim.x + threadIdx.x;
-  if (p >= T * K) return;
-  const int e = idx[p];
-  slot_w[p] = (aff && e >= 0 && e < E) ? aff[(long long)(p / K) * E + e] : (aff ? 0.0f : 1.0f);
-}
-
-__global__ void copy_slot_weights(const float* src, int n, float* dst) {
-  const int p = blockIdx.x * blockDim.x + threadIdx.x;
-  if (p < n) dst[p] = src[p];
-}
-
 // Per-wave K slice of the frag gate/up GEMM (two row blocks per wave).
 int gate_up_kw(int H, int I, int gmax) { return choose_kw(H, 256, (long long)(I / 16) * gmax); }
 
@@ -310,12 +297,17 @@ int moe_core(const uint16_t* hidden, const void* gate_up, const void* down, cons
              const RouterArgs* sel = nullptr, unsigned* fused_flags = nullptr,
              unsigned* fused_err = nullptr, uint16_t* poll_h = nullptr,
              const uint16_t* hn_r = nullptr, const uint16_t* hn_gamma = nullptr,
-             bool x_mx_ready = false) {
+             bool x_mx_ready = false, MoeBegin begin = MoeBegin{}) {
   if (sel && (idx || wfmt || tiled)) return MKD_ERR_INVALID;
   if (fused_flags && !sel) return MKD_ERR_INVALID;
-  if (idx)  // otherwise the router stage already built the expert groups
+  if (idx) {  // otherwise the router stage already built the expert groups
+    if ((wfmt == MKD_MX_E4M3 || wfmt == MKD_MX_E2M1) && !x_mx_ready) {   // the hidden rows' MXFP8 form
+      begin.x = hidden; begin.H = H; begin.mx_kpad = mx_pad(H); begin.xq = w.xq; begin.xs = w.xs;
+      x_mx_ready = true;
+    }
     MKD_TRY(moe_route_launch(idx, T, K, E, w.n_groups, w.grp_expert, w.grp_count, w.grp_offset,
-                             w.pair_token, w.pair_slot, s, w.route_off), "moe_route");
+                             w.pair_token, w.pair_slot, s, w.route_off, &begin), "moe_route");
+  }
   const int gmax = E < T * K ? E : T * K;
   if (wfmt == MKD_FP8_E4M3) {
     // e4m3 experts (FP8 ROW / STATIC): bf16 activations, per-column dequantisation
@@ -701,22 +693,18 @@ int moe_entry(const mkd_moe_args* p, void* workspace, size_t workspace_bytes, vo
   MoeWs w = carve_moe(c, p->T, p->H, p->E, p->I, p->K);
   MKD_REQUIRE(c.ok, MKD_ERR_WORKSPACE, "moe_tkg: workspace %zu < %zu bytes", workspace_bytes, c.used);
   hipStream_t s = static_cast<hipStream_t>(stream);
-  const int TK = p->T * p->K;
-  if (p->slot_weights) {
-    hipLaunchKernelGGL(copy_slot_weights, dim3((TK + 255) / 256), dim3(256), 0, s, p->slot_weights, TK, w.slot_w);
-  } else {
-    hipLaunchKernelGGL(gather_slot_weights, dim3((TK + 255) / 256), dim3(256), 0, s,
-                       p->scaling_mode == MKD_SCALE_POST ? p->expert_affinities : nullptr,
-                       p->expert_index, p->T, p->E, p->K, w.slot_w);
-  }
-  MKD_TRY(hipGetLastError(), "slot weights");
+  MoeBegin begin = {};
+  begin.slot_w = w.slot_w;
+  begin.slot_src = p->slot_weights;
+  begin.aff = p->scaling_mode == MKD_SCALE_POST ? p->expert_affinities : nullptr;
   return moe_core(static_cast<const uint16_t*>(p->hidden), p->gate_up_packed, p->down_packed,
                   p->expert_index, w.slot_w, static_cast<const uint16_t*>(p->gate_up_bias),
                   static_cast<const uint16_t*>(p->down_bias),
                   static_cast<const uint16_t*>(p->residual), static_cast<uint16_t*>(p->output),
                   p->output_f32, p->T, p->H, p->E, p->I, p->K, p->activation, p->alpha,
                   p->gate_hi, p->gate_lo, p->up_hi, p->up_lo, p->round_qwen, w, s, true,
-                  p->weight_format, p->gate_up_scales, p->down_scales, tiled);
+                  p->weight_format, p->gate_up_scales, p->down_scales, tiled, nullptr, nullptr, nullptr, nullptr, nullptr,
+                  nullptr, false, begin);
 }
 }  // namespace
 

@@ -544,9 +544,19 @@ constexpr int kRouteChunk = 2048;          // slots per placing block, at least
 constexpr int kRouteMaxChunks = 64;
 constexpr int kRouteChunkCounts = 8192;    // per-chunk counts: chunks x E <= this
 int moe_route_chunk(int TK, int E);        // slots per chunk, 0 = the one-block form
+// What else an expert call's first launch does (moe_route_kernel): the slots'
+// weights (slot_w; from `aff` [T, E] by expert id, `slot_src` [T K], or 1 with
+// neither) and the hidden rows' MXFP8 form (xq / xs of x [T, H]).  Null: skipped.
+struct MoeBegin {
+  float* slot_w;
+  const float *aff, *slot_src;
+  const uint16_t* x;
+  int H, mx_kpad;
+  uint8_t *xq, *xs;
+};
 hipError_t moe_route_launch(const int* idx, int T, int K, int E, int* n_groups, int* grp_expert,
                             int* grp_count, int* grp_offset, int* pair_token, int* pair_slot,
-                            hipStream_t s, int* chunk_off = nullptr);
+                            hipStream_t s, int* chunk_off = nullptr, const MoeBegin* begin = nullptr);
 hipError_t moe_finalize_launch(const float* ybuf, int T, int K, int H, const uint16_t* resid,
                                uint16_t* out, float* out_f32, hipStream_t s);
 

@@ -18,6 +18,7 @@
 //   bf16 residual add.
 #include "common.h"
 #include "mkd_internal.h"
+#include "mx_codec.h"
 #include "router_select.h"
 #include "launch_rules.h"
 
@@ -71,11 +72,28 @@ hipError_t router_select_multi_launch(const RouterArgs& a, hipStream_t s) {
 }
 
 // ---------------------------------------------------------------------------
+// Slot p's weight: its token's affinity for expert e (0 for an id outside the
+// experts), a given weight, or 1.
+MKD_DEV float slot_weight(const MoeBegin& m, int p, int e, int K, int E) {
+  if (m.slot_src) return m.slot_src[p];
+  if (!m.aff) return 1.0f;
+  return e >= 0 && e < E ? m.aff[(long long)(p / K) * E + e] : 0.0f;
+}
+
+// Block 0 routes; with MoeBegin it also fills the slot weights (below the split
+// form), and the blocks after it quantise the hidden rows to MXFP8 -- work of the
+// expert operator that needs no order among itself, as one launch instead of three.
 __global__ void __launch_bounds__(1024)
 moe_route_kernel(const int* __restrict__ idx, int T, int K, int E, int* __restrict__ n_groups,
                  int* __restrict__ grp_expert, int* __restrict__ grp_count,
                  int* __restrict__ grp_offset, int* __restrict__ pair_token,
-                 int* __restrict__ pair_slot, int cs, int nc, int* __restrict__ chunk_off) {
+                 int* __restrict__ pair_slot, int cs, int nc, int* __restrict__ chunk_off, MoeBegin mb) {
+  if (blockIdx.x > 0) {
+    const long long it = (blockIdx.x - 1) * 1024LL + threadIdx.x;
+    if (it < (long long)T * (mb.mx_kpad / 8))
+      mx_quant_rows_item<false>(mb.x, it, mb.H, mb.H, mb.xq, mb.xs, mb.mx_kpad);
+    return;
+  }
   __shared__ int cnt[kMaxE], off[kMaxE], cursor[kMaxE];
   __shared__ int wtot[16];
   // split form (chunk_off set): per-chunk counts [nc][E] of the cs-slot chunks
@@ -96,6 +114,13 @@ moe_route_kernel(const int* __restrict__ idx, int T, int K, int E, int* __restri
     for (int u = 0; u < CH; ++u) {
       const int p = p0 + u * nt + tid;
       ev[u] = p < TK ? idx[p] : -1;
+    }
+    if (mb.slot_w && !split) {   // (the split form: moe_route_scatter_kernel)
+#pragma unroll
+      for (int u = 0; u < CH; ++u) {
+        const int p = p0 + u * nt + tid;
+        if (p < TK) mb.slot_w[p] = slot_weight(mb, p, ev[u], K, E);
+      }
     }
 #pragma unroll
     for (int u = 0; u < CH; ++u) {
@@ -179,7 +204,7 @@ moe_route_kernel(const int* __restrict__ idx, int T, int K, int E, int* __restri
 __global__ void __launch_bounds__(256)
 moe_route_scatter_kernel(const int* __restrict__ idx, int TK, int K, int E, int cs,
                          const int* __restrict__ chunk_off, int* __restrict__ pair_token,
-                         int* __restrict__ pair_slot) {
+                         int* __restrict__ pair_slot, MoeBegin mb) {
   __shared__ int base_s[kMaxE], cursor[kMaxE];
   constexpr int CH = 8;
   const int tid = threadIdx.x, nt = (int)blockDim.x;
@@ -196,6 +221,13 @@ moe_route_scatter_kernel(const int* __restrict__ idx, int TK, int K, int E, int 
       const int p = p0 + u * nt + tid;
       ev[u] = p < p_hi ? idx[p] : -1;
     }
+    if (mb.slot_w) {
+#pragma unroll
+      for (int u = 0; u < CH; ++u) {
+        const int p = p0 + u * nt + tid;
+        if (p < p_hi) mb.slot_w[p] = slot_weight(mb, p, ev[u], K, E);
+      }
+    }
 #pragma unroll
     for (int u = 0; u < CH; ++u) {
       const int e = ev[u];
@@ -209,26 +241,34 @@ moe_route_scatter_kernel(const int* __restrict__ idx, int TK, int K, int E, int 
 }
 
 // ---------------------------------------------------------------------------
+// Eight expert rows' loads are in flight before the first is added (8192 tokens x 8
+// rows of 2048: 117 us one row at a time).
 __global__ void __launch_bounds__(256)
 moe_finalize_kernel(const float* __restrict__ ybuf, int K, int H, const uint16_t* __restrict__ resid,
                     uint16_t* __restrict__ out, float* __restrict__ out_f32) {
   const int t = blockIdx.y;
-  const int i = (blockIdx.x * 256 + threadIdx.x) * 4;
+  const int i = (blockIdx.x * blockDim.x + threadIdx.x) * 4;
   if (i >= H) return;
+  const float* y0 = ybuf + (long long)t * K * H + i;
+  const long long o0 = (long long)t * H + i;
   f32x4_t s = {0.f, 0.f, 0.f, 0.f};
-  for (int k = 0; k < K; ++k) {
-    const f32x4_t y = *reinterpret_cast<const f32x4_t*>(ybuf + ((long long)t * K + k) * H + i);
-    s += y;
+  for (int k0 = 0; k0 < K; k0 += 8) {
+    f32x4_t y[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) y[k] = *reinterpret_cast<const f32x4_t*>(y0 + (long long)min(k0 + k, K - 1) * H);
+#pragma unroll
+    for (int k = 0; k < 8; ++k)
+      if (k0 + k < K) s += y[k];
   }
-  if (out_f32) *reinterpret_cast<f32x4_t*>(out_f32 + (long long)t * H + i) = s;
+  if (out_f32) *reinterpret_cast<f32x4_t*>(out_f32 + o0) = s;
   if (out) {
     float o[4];
     for (int j = 0; j < 4; ++j) o[j] = rbf(s[j]);
     if (resid) {
-      const uint2 r = *reinterpret_cast<const uint2*>(resid + (long long)t * H + i);
+      const uint2 r = *reinterpret_cast<const uint2*>(resid + o0);
       o[0] += bf_lo(r.x); o[1] += bf_hi(r.x); o[2] += bf_lo(r.y); o[3] += bf_hi(r.y);
     }
-    *reinterpret_cast<uint2*>(out + (long long)t * H + i) = uint2{pack2bf(o[0], o[1]), pack2bf(o[2], o[3])};
+    *reinterpret_cast<uint2*>(out + o0) = uint2{pack2bf(o[0], o[1]), pack2bf(o[2], o[3])};
   }
 }
 
@@ -420,18 +460,21 @@ int moe_route_chunk(int TK, int E) {
 
 hipError_t moe_route_launch(const int* idx, int T, int K, int E, int* n_groups, int* grp_expert,
                             int* grp_count, int* grp_offset, int* pair_token, int* pair_slot,
-                            hipStream_t s, int* chunk_off) {
+                            hipStream_t s, int* chunk_off, const MoeBegin* begin) {
   if (E > kMaxE || T < 0 || K < 1) return hipErrorInvalidValue;
+  const MoeBegin mb = begin ? *begin : MoeBegin{};
+  if (mb.xq && (!mb.x || !mb.xs || mb.H % 32 || mb.mx_kpad % 128 || mb.mx_kpad < mb.H)) return hipErrorInvalidValue;
   const int TK = T * K;
   const int cs = chunk_off ? moe_route_chunk(TK, E) : 0;
   const int nc = cs ? (TK + cs - 1) / cs : 0;
-  hipLaunchKernelGGL(moe_route_kernel, dim3(1), dim3(1024), 0, s, idx, T, K, E, n_groups,
+  const long long nq = mb.xq ? ((long long)T * (mb.mx_kpad / 8) + 1023) / 1024 : 0;
+  hipLaunchKernelGGL(moe_route_kernel, dim3((unsigned)(1 + nq)), dim3(1024), 0, s, idx, T, K, E, n_groups,
                      grp_expert, grp_count, grp_offset, pair_token, pair_slot, cs ? cs : 1, nc,
-                     cs ? chunk_off : nullptr);
+                     cs ? chunk_off : nullptr, mb);
   if (hipError_t e = hipGetLastError()) return e;
   if (cs)
     hipLaunchKernelGGL(moe_route_scatter_kernel, dim3(nc), dim3(256), 0, s, idx, TK, K, E, cs,
-                       chunk_off, pair_token, pair_slot);
+                       chunk_off, pair_token, pair_slot, mb);
   return hipGetLastError();
 }
 

@@ -1,7 +1,7 @@
 // MX (OCP Microscaling v1.0) expert path for gfx950: MXFP8 / MXFP4 weights,
 // MXFP8 activations, v_mfma_scale_f32_16x16x128_f8f6f4.
 //
-// Quantisation (mx_quantize_kernel): blocks of 32 consecutive elements along K
+// Quantisation (mx_quantize_*_kernel): blocks of 32 consecutive elements along K
 // share one E8M0 scale X = 2^(floor(log2 amax) - emax_elem) (byte = exponent
 // + 127, clamped to [0, 254]; an all-zero block gets byte 0); each element is
 // v / X rounded to nearest-even in the element format and saturated to its
@@ -40,14 +40,23 @@ namespace mkd {
 typedef __attribute__((__vector_size__(8 * sizeof(int)))) int i32x8_t;
 
 // ---------------------------------------------------------------------------
-// Quantisation: one thread per 32-element block.  codes row stride: K_pad bytes
-// (e4m3) or K_pad/2 bytes (e2m1, two per byte, low nibble first); scales row
-// stride K_pad/32.  Blocks at k >= K are written as zeros.
+// Quantisation.  codes row stride: K_pad bytes (e4m3) or K_pad/2 bytes (e2m1, two
+// per byte, low nibble first); scales row stride K_pad/32.  Blocks at k >= K are
+// written as zeros.  E4M3 (activations on every call): four lanes per 32-element
+// block.  E2M1 (weights, once): one thread per block.
 // ---------------------------------------------------------------------------
-template <int FMT, bool XF32>
-__global__ void mx_quantize_kernel(const void* __restrict__ x, int rows, int K, int ldx,
-                                   uint8_t* __restrict__ codes, uint8_t* __restrict__ scales,
-                                   int K_pad) {
+template <bool XF32>
+__global__ void __launch_bounds__(256) mx_quantize_e4m3_kernel(const void* __restrict__ x, int rows, int K, int ldx,
+                                                               uint8_t* __restrict__ codes,
+                                                               uint8_t* __restrict__ scales, int K_pad) {
+  const long long it = blockIdx.x * 256LL + threadIdx.x;   // (K_pad / 8 is a multiple of 16: whole quads)
+  if (it < (long long)rows * (K_pad / 8)) mx_quant_rows_item<XF32>(x, it, K, ldx, codes, scales, K_pad);
+}
+
+template <bool XF32>
+__global__ void mx_quantize_e2m1_kernel(const void* __restrict__ x, int rows, int K, int ldx,
+                                        uint8_t* __restrict__ codes, uint8_t* __restrict__ scales,
+                                        int K_pad) {
   const int nblk = K_pad / 32;
   const long long idx = blockIdx.x * (long long)blockDim.x + threadIdx.x;
   if (idx >= (long long)rows * nblk) return;
@@ -80,31 +89,17 @@ __global__ void mx_quantize_kernel(const void* __restrict__ x, int rows, int K, 
   float amax = 0.f;
 #pragma unroll
   for (int j = 0; j < 32; ++j) amax = fmaxf(amax, fabsf(v[j]));
-  const uint32_t sb = mx_scale_byte<FMT>(amax);
+  const uint32_t sb = mx_scale_byte<MX_E2M1>(amax);
   const int sh = 127 - (int)sb;
-  if (FMT == MX_E4M3) {
-    u32x4_t o[2];
+  u32x4_t o;
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      uint32_t d = 0;
+  for (int j = 0; j < 4; ++j) {
+    uint32_t d = 0;
 #pragma unroll
-      for (int h = 0; h < 4; ++h) d |= mx_encode<FMT>(ldexpf(v[4 * j + h], sh)) << (8 * h);
-      o[j >> 2][j & 3] = d;
-    }
-    uint8_t* c = codes + (long long)r * K_pad + b * 32;
-    st16(c, o[0]);
-    st16(c + 16, o[1]);
-  } else {
-    u32x4_t o;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      uint32_t d = 0;
-#pragma unroll
-      for (int h = 0; h < 8; ++h) d |= mx_encode<FMT>(ldexpf(v[8 * j + h], sh)) << (4 * h);
-      o[j] = d;
-    }
-    st16(codes + (long long)r * (K_pad / 2) + b * 16, o);
+    for (int h = 0; h < 8; ++h) d |= mx_encode<MX_E2M1>(ldexpf(v[8 * j + h], sh)) << (4 * h);
+    o[j] = d;
   }
+  st16(codes + (long long)r * (K_pad / 2) + b * 16, o);
   scales[(long long)r * nblk + b] = (uint8_t)sb;
 }
 
@@ -391,12 +386,11 @@ __global__ void __launch_bounds__(512) gemm_mx_kernel(GemmArgs a) {
 hipError_t mx_quantize_launch(const void* x, bool x_f32, int rows, int K, int ldx, int fmt,
                               uint8_t* codes, uint8_t* scales, int K_pad, hipStream_t s) {
   if (rows <= 0 || K <= 0 || K % 32 || K_pad < K || K_pad % 128) return hipErrorInvalidValue;
-  const long long n = (long long)rows * (K_pad / 32);
-  const int threads = 256;
-  const unsigned blocks = (unsigned)((n + threads - 1) / threads);
-#define MKD_Q(F, X) hipLaunchKernelGGL((mx_quantize_kernel<F, X>), dim3(blocks), dim3(threads), 0, s, x, rows, K, ldx, codes, scales, K_pad)
-  if (fmt == MX_E4M3) { if (x_f32) MKD_Q(MX_E4M3, true); else MKD_Q(MX_E4M3, false); }
-  else if (fmt == MX_E2M1) { if (x_f32) MKD_Q(MX_E2M1, true); else MKD_Q(MX_E2M1, false); }
+  const long long n = (long long)rows * (fmt == MX_E4M3 ? K_pad / 8 : K_pad / 32);
+  const dim3 grid((unsigned)((n + 255) / 256)), block(256);
+#define MKD_Q(KERN, X) hipLaunchKernelGGL((KERN<X>), grid, block, 0, s, x, rows, K, ldx, codes, scales, K_pad)
+  if (fmt == MX_E4M3) { if (x_f32) MKD_Q(mx_quantize_e4m3_kernel, true); else MKD_Q(mx_quantize_e4m3_kernel, false); }
+  else if (fmt == MX_E2M1) { if (x_f32) MKD_Q(mx_quantize_e2m1_kernel, true); else MKD_Q(mx_quantize_e2m1_kernel, false); }
   else return hipErrorInvalidValue;
 #undef MKD_Q
   return hipGetLastError();

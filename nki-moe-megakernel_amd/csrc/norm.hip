@@ -114,22 +114,13 @@ __global__ void __launch_bounds__(kNormThreads) rmsnorm_kernel(NormArgs a) {
         *reinterpret_cast<f32x4_t*>(op + 4) = f32x4_t{y[4], y[5], y[6], y[7]};
       }
       if (a.mx_codes) {
-        // the block's amax over the four threads tid & ~3 .. +3 (H % 32 == 0:
-        // all four are in range together)
-        float q[8], amax = 0.f;
+        // a block is the four threads tid & ~3 .. +3 (H % 32 == 0: all four are
+        // in range together)
+        float q[8];
 #pragma unroll
-        for (int j = 0; j < 8; ++j) {
-          q[j] = rbf(y[j]);
-          amax = fmaxf(amax, fabsf(q[j]));
-        }
-        amax = fmaxf(amax, __shfl_xor(amax, 1, 64));
-        amax = fmaxf(amax, __shfl_xor(amax, 2, 64));
-        const uint32_t sb = mx_scale_byte<MX_E4M3>(amax);
-        const int sh = 127 - (int)sb;
-        uint2 c = {0u, 0u};
-#pragma unroll
-        for (int j = 0; j < 8; ++j)
-          (j < 4 ? c.x : c.y) |= mx_encode<MX_E4M3>(ldexpf(q[j], sh)) << (8 * (j & 3));
+        for (int j = 0; j < 8; ++j) q[j] = rbf(y[j]);
+        uint32_t sb;
+        const uint2 c = mx_quant8_e4m3(q, sb);
         *reinterpret_cast<uint2*>(a.mx_codes + (long long)row * a.mx_kpad + i) = c;
         if ((tid & 3) == 0) a.mx_scales[(long long)row * (a.mx_kpad / 32) + i / 32] = (uint8_t)sb;
       }
