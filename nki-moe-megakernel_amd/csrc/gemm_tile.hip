@@ -4,7 +4,7 @@
 //
 //   Y[t, n] = sum_k X[row(t), k] * W_e[n, k]   for the tokens t of expert e
 //
-// Block tile 256 weight rows x up to 128 tokens, 4 waves, two blocks per CU.  Wave
+// Block tile 256 weight rows x up to 160 tokens, 4 waves, two blocks per CU.  Wave
 // w owns rows 64 w .. +64 (four 16-row blocks) of every token of the tile: it
 // loads its weight fragments straight into registers (the packed layout is MFMA
 // operand order, 1 KiB contiguous per fragment, each read by one wave of the
@@ -21,9 +21,11 @@
 // one's group scan, first stage and epilogue (13 of the former block's 60 us)
 // with the other's k loop.
 //
-// The inner loop is compiled for 32, 64, 96 and 128 tokens and picked by the
-// tile's live tokens, so a group's last tile (or a small expert's only one)
-// multiplies at most 31 absent tokens.
+// The inner loop is compiled for 32 .. 160 tokens and picked by the tile's live
+// tokens.  A group of c tokens is cut into ceil(c / 160) equal tiles: with 128-token
+// tiles a batch of ~128 tokens per expert left half the experts a second tile of a
+// few tokens that streamed the expert's weights again (2048 tokens routed at random:
+// gate/up 187 us against 143 at exactly 128 per expert).
 //
 // Epilogues: EPI_SWIGLU_BF16 (gate / up row blocks interleaved in the packing,
 // so both halves of a pair sit in the same wave) and EPI_SCALE_F32 (affinity
@@ -38,22 +40,17 @@ namespace mkd {
 namespace {
 
 constexpr int kTileRows = 256;           // packed weight rows per block
-constexpr int kTileTok = 128;            // tokens per block (at most)
+constexpr int kTileTok = 160;            // tokens per block (at most)
 constexpr int kRB = kTileRows / 16;      // row blocks per block (16)
 constexpr int kNW = 4;                   // waves; each owns kRB / kNW = 4 row blocks
 constexpr int kStages = 4;               // LDS ring of 64-k token stages
 constexpr int kStageTokBytes = 128;      // one token's 64 k of a stage
 constexpr int kRingBytes = kStages * kTileTok * kStageTokBytes;
-// the fp32 epilogue stages half of the output tile in LDS, [128 tokens][128 + 4
-// rows] (the 4 floats of padding spread a lane group's 16 rows over the banks),
-// then the block's output row indices
-constexpr int kStgLd = 132;
-constexpr int kStgBytes = kTileTok * kStgLd * 4 + kTileTok * 4;
-// the SwiGLU epilogue stages the whole h tile, [128 tokens][128 + 8 columns]
+// the SwiGLU epilogue stages the whole h tile, [160 tokens][128 + 8 columns]
 // bf16 (the padding shifts each token row by 4 banks), then the row indices
 constexpr int kHsLd = 136;
-static_assert(kTileTok * kHsLd * 2 + kTileTok * 4 <= kStgBytes, "h staging fits the fp32 staging area");
-constexpr int kLdsBytes = kRingBytes > kStgBytes ? kRingBytes : kStgBytes;
+constexpr int kLdsBytes = kRingBytes;
+static_assert(kTileTok * kHsLd * 2 + kTileTok * 4 <= kRingBytes, "h staging fits the ring");
 static_assert(2 * kLdsBytes <= 160 * 1024, "two blocks per CU");
 
 // s_waitcnt with only vmcnt = n (expcnt / lgkmcnt left at their maxima); gfx9
@@ -92,17 +89,19 @@ struct IntC {
 struct TileJob {
   const uint16_t* wp;      // the expert's packed weights
   int nb0;                 // first row block
-  int count, base, t0;     // the group's tokens, its first pair, the tile's first token
+  int count, base, t0;     // the tile's end and first token in the group, the group's first pair
   int expert, kq;          // expert (bias), K slice
   int s0, S;               // first 32-wide k step, k steps
 };
 
-// The k loop and epilogue for tiles of at most 16 * WT tokens (WT even); PAIRS:
-// the k steps are a multiple of 4.
+// The k loop and epilogue for tiles of at most 16 * WT tokens; PAIRS: the k steps
+// are a multiple of 4.  Weight fragments are loaded four k steps ahead, two where
+// the accumulators leave no registers for more (WT > 8).
 template <int EPI, int WT, bool PAIRS>
 MKD_DEV void tile_body(const GemmArgs& a, const TileJob& jb, char* lds) {
-  constexpr int C = WT / 2;              // 8-token copies per wave per stage
-  constexpr int HT = WT / 2;             // token tiles per half step
+  constexpr int C = (WT + 1) / 2;        // 8-token copies per wave per stage
+  constexpr int H0 = (WT + 1) / 2, H1 = WT / 2;   // token tiles of a step's halves
+  constexpr int AD = WT > 8 ? 2 : 4;     // weight k steps in flight
   const int tid = threadIdx.x, lane = tid & 63;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int KB = a.K / 32, NB = (a.N + 15) / 16;
@@ -120,7 +119,7 @@ MKD_DEV void tile_body(const GemmArgs& a, const TileJob& jb, char* lds) {
   int voff[C];
 #pragma unroll
   for (int j = 0; j < C; ++j) {
-    const int t = (w + kNW * j) * 8 + (lane >> 3);
+    const int t = (w + kNW * j) * 8 + (lane >> 3);      // (past 16 WT: into unused slots)
     const int tc = min(jb.t0 + t, jb.count - 1);        // absent: any valid row
     const int row = a.pair_row ? a.pair_row[jb.base + tc] : jb.base + tc;
     voff[j] = (row * a.ldx + jb.s0 * 32) * 2 + (((lane & 7) ^ ((t >> 1) & 7)) << 4);
@@ -143,7 +142,7 @@ MKD_DEV void tile_body(const GemmArgs& a, const TileJob& jb, char* lds) {
 #pragma unroll
   for (int i = 0; i < 4; ++i)            // rows past N: any valid block
     aoff[i] = __builtin_amdgcn_readfirstlane((min(jb.nb0 + 4 * w + i, NB - 1) * KB + jb.s0) * 1024);
-  u32x4_t af[4][4];                      // [k step % 4][row block]
+  u32x4_t af[AD][4];                     // [k step % AD][row block]
   auto load_a = [&](u32x4_t (&f)[4], int step) {
     const int vo = lane * 16 | (step < S ? 0 : -1);
     issue_fence();
@@ -153,11 +152,12 @@ MKD_DEV void tile_body(const GemmArgs& a, const TileJob& jb, char* lds) {
   };
   // ---- operand reads: token tile j, step h of the stage in ring slot s % 4 ----
   const int rd = (lane & 15) * kStageTokBytes + (((lane >> 4) ^ ((lane >> 1) & 7)) << 4);
-  auto read_b = [&](u32x4_t (&b)[HT], int s, int h, int half) {
+  auto read_b = [&](auto& b, int s, int h, int j0) {
+    constexpr int n = sizeof(b) / sizeof(b[0]);
     const char* st = lds + (s & (kStages - 1)) * (kTileTok * kStageTokBytes) + (rd ^ (h * 64));
 #pragma unroll
-    for (int j = 0; j < HT; ++j)
-      b[j] = *reinterpret_cast<const u32x4_t*>(st + (half * HT + j) * 16 * kStageTokBytes);
+    for (int j = 0; j < n; ++j)
+      b[j] = *reinterpret_cast<const u32x4_t*>(st + (j0 + j) * 16 * kStageTokBytes);
     __builtin_amdgcn_sched_barrier(0);
   };
   f32x4_t acc[4][WT];
@@ -165,17 +165,19 @@ MKD_DEV void tile_body(const GemmArgs& a, const TileJob& jb, char* lds) {
   for (int i = 0; i < 4; ++i)
 #pragma unroll
     for (int j = 0; j < WT; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-  auto mul = [&](const u32x4_t (&f)[4], const u32x4_t (&b)[HT], int half) {
+  auto mul = [&](const u32x4_t (&f)[4], const auto& b, int j0) {
+    constexpr int n = sizeof(b) / sizeof(b[0]);
 #pragma unroll
-    for (int j = 0; j < HT; ++j)
+    for (int j = 0; j < n; ++j)
 #pragma unroll
-      for (int i = 0; i < 4; ++i) acc[i][half * HT + j] = mfma16x16x32(f[i], b[j], acc[i][half * HT + j]);
+      for (int i = 0; i < 4; ++i) acc[i][j0 + j] = mfma16x16x32(f[i], b[j], acc[i][j0 + j]);
     __builtin_amdgcn_sched_barrier(0);
   };
 
-  // Issue order of a wave's vector-memory operations (the waits count them):
-  //   prologue: copies(0) copies(1) A(0) copies(2) A(1)
-  //   stage s:  A0(s+2) [barrier] copies(s+3) A1(s+2)      (A0 / A1: 4 loads each)
+  // Issue order of a wave's vector-memory operations (the waits count them); A0 / A1
+  // are the 4 loads of a stage's first / second k step, d = AD / 2 stages ahead:
+  //   prologue: copies(0) copies(1) A(0) copies(2) [A(1) if d = 2]
+  //   stage s:  A0(s+d) [barrier] copies(s+3) A1(s+d)
   // Past the last stage they are issued with an offset past the buffer (no memory
   // access, zeros), so the counts and the compiler's own waits on the weight
   // registers stay exact without branches.  In the middle of stage s every wave
@@ -184,36 +186,37 @@ MKD_DEV void tile_body(const GemmArgs& a, const TileJob& jb, char* lds) {
   //    next barrier);
   //  * every wave's reads of stage s - 1 are complete (consumed by its MFMAs),
   //    so that ring slot takes stage s + 3.
-  // Operations issued after copies(s + 1): A1(s) A0(s+1) copies(s+2) A1(s+1)
-  // A0(s+2) = 16 + C (the prologue's order adds to that, so the wait holds there
-  // too).
+  // Operations issued after copies(s + 1): A1 A0 copies(s+2) A1 A0 = 16 + C from
+  // stage 2 on, and at least 12 + C in stages 0 and 1.
   issue(0);
   issue(1);
   load_a(af[0], 0);
   load_a(af[1], 1);
   issue(2);
-  load_a(af[2], 2);
-  load_a(af[3], 3);
-  wait_vmcnt<16 + 2 * C>();              // copies(0) landed: 2 C + 16 issued after them
+  if (AD == 4) {
+    load_a(af[AD - 2], 2);
+    load_a(af[AD - 1], 3);
+  }
+  wait_vmcnt<4 * AD + 2 * C>();          // copies(0) landed: that many issued after them
   block_barrier();
-  u32x4_t b0[HT], b1[HT];
+  u32x4_t b0[H0], b1[H1];
   read_b(b0, 0, 0, 0);
   auto first = [&](int s, u32x4_t (&f0)[4]) {
-    read_b(b1, s, 0, 1);
+    read_b(b1, s, 0, H0);
     mul(f0, b0, 0);
     read_b(b0, s, 1, 0);
-    mul(f0, b1, 1);
+    mul(f0, b1, H0);
   };
   auto second = [&](int s, u32x4_t (&f0)[4], u32x4_t (&f1)[4]) {
-    load_a(f0, 2 * s + 4);
-    wait_vmcnt<16 + C>();
+    load_a(f0, 2 * s + AD);
+    wait_vmcnt<12 + C>();
     block_barrier();
     issue(s + 3);
-    read_b(b1, s, 1, 1);
+    read_b(b1, s, 1, H0);
     mul(f1, b0, 0);
     read_b(b0, s + 1, 0, 0);             // (past the last stage: unused)
-    mul(f1, b1, 1);
-    load_a(f1, 2 * s + 5);
+    mul(f1, b1, H0);
+    load_a(f1, 2 * s + 1 + AD);
   };
   // PAIRS (S a multiple of 4, every shape of the two models): one exit, so that the
   // compiler's counts at the loop head are those of a full turn.  Otherwise the
@@ -222,8 +225,8 @@ MKD_DEV void tile_body(const GemmArgs& a, const TileJob& jb, char* lds) {
     for (int s = 0; s < NS; s += 2) {
       first(s, af[0]);
       second(s, af[0], af[1]);
-      first(s + 1, af[2]);
-      second(s + 1, af[2], af[3]);
+      first(s + 1, af[AD - 2]);
+      second(s + 1, af[AD - 2], af[AD - 1]);
     }
   } else {
     for (int s = 0;; s += 2) {
@@ -231,9 +234,9 @@ MKD_DEV void tile_body(const GemmArgs& a, const TileJob& jb, char* lds) {
       if (2 * s + 1 == S) break;
       second(s, af[0], af[1]);
       if (2 * s + 2 == S) break;
-      first(s + 1, af[2]);
+      first(s + 1, af[AD - 2]);
       if (2 * s + 3 == S) break;
-      second(s + 1, af[2], af[3]);
+      second(s + 1, af[AD - 2], af[AD - 1]);
       if (2 * s + 4 == S) break;
     }
   }
@@ -300,65 +303,57 @@ MKD_DEV void tile_body(const GemmArgs& a, const TileJob& jb, char* lds) {
   } else {   // EPI_SCALE_F32
     // (K slices: the bias joins the first slice's partial)
     const uint16_t* bp = a.bias && jb.kq == 0 ? a.bias + (long long)jb.expert * a.bias_group_stride : nullptr;
-    // The tile goes out through LDS, half (128 rows) at a time: the waves of
-    // that half store their scaled accumulators as [token][row], then every
-    // thread writes 16 contiguous bytes of a token's 512-byte row segment --
-    // directly, a store instruction wrote 64 bytes into each of 16 scattered
-    // output rows, and the stores took ~40 % of the down projection's time.
-    float* stg = reinterpret_cast<float*>(lds);
-    int* orow_s = reinterpret_cast<int*>(stg + kTileTok * kStgLd);
-    // all affinities up front (y is float too, so loads among the stores could
-    // not be moved past them)
-    float sc[WT];
+    // Each wave turns its 64 rows x 16 tokens through its own 4 KiB of LDS and stores
+    // 256 contiguous bytes per token (16 lanes x 16 bytes), with no barrier among
+    // the waves.  Straight from the registers a store covers 64 bytes of each of 16
+    // rows: 2048 tokens 119 instead of 112 us.  The grouped rows (T K of them) are
+    // read back once, by the finalize: non-temporal, 2.7 % of moe_prefill at 8192
+    // tokens; the dense rows are the next kernel's input.
+    constexpr int kLd = 68;                           // 64 rows + 4 floats of padding
+    float* stg = reinterpret_cast<float*>(lds) + w * 16 * kLd;
+    __syncthreads();                                  // every wave is past its last operand reads
+    float* ybase = static_cast<float*>(a.y) + jb.kq * a.part_stride;
+    const int n0 = (jb.nb0 + w * 4) * 16, n = n0 + (lane & 15) * 4;
+    // the output rows and scales of tokens lane, lane + 64, lane + 128 of the tile
+    int orow[(WT + 3) / 4];
+    float osc[(WT + 3) / 4];
+#pragma unroll
+    for (int k = 0; k < (WT + 3) / 4; ++k) {
+      const int t = min(jb.t0 + 64 * k + lane, jb.count - 1);
+      orow[k] = a.pair_out_row ? a.pair_out_row[jb.base + t] : jb.base + t;
+      osc[k] = a.pair_scale ? a.pair_scale[orow[k]] : 1.0f;
+    }
+    float bb[4] = {0.f, 0.f, 0.f, 0.f};               // this lane's four rows as stored
+    if (bp) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) bb[e] = n + e < a.N ? bf2f(bp[n + e]) : 0.f;
+    }
 #pragma unroll
     for (int j = 0; j < WT; ++j) {
-      const int tc = min(jb.t0 + j * 16 + (lane & 15), jb.count - 1);
-      sc[j] = a.pair_scale ? a.pair_scale[a.pair_out_row ? a.pair_out_row[jb.base + tc] : jb.base + tc] : 1.0f;
-    }
-    int orow = 0;
-    if (tid < NT) {
-      const int tc = min(jb.t0 + tid, jb.count - 1);
-      orow = a.pair_out_row ? a.pair_out_row[jb.base + tc] : jb.base + tc;
-    }
-    __syncthreads();                     // every wave is past its last operand reads
-    if (tid < NT) orow_s[tid] = orow;
-    float* ybase = static_cast<float*>(a.y) + jb.kq * a.part_stride;
 #pragma unroll
-    for (int half = 0; half < 2; ++half) {
-      if (w >> 1 == half) {
+      for (int i = 0; i < 4; ++i)
+        *reinterpret_cast<f32x4_t*>(stg + (lane & 15) * kLd + i * 16 + q4) = acc[i][j];
+      wave_lds_sync();
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const int n = (jb.nb0 + w * 4 + i) * 16 + q4;
-          float bb[4] = {0.f, 0.f, 0.f, 0.f};
-          if (bp) {
+      for (int u = 0; u < 4; ++u) {
+        const int tl = 4 * u + (lane >> 4), tt = j * 16 + tl;   // token of the 16, of the tile
+        f32x4_t v = *reinterpret_cast<const f32x4_t*>(stg + tl * kLd + (lane & 15) * 4);
+        const int row = __shfl(orow[j / 4], tt & 63, 64);
+        const float sc = __shfl(osc[j / 4], tt & 63, 64);
+        if (jb.t0 + tt >= jb.count) continue;
 #pragma unroll
-            for (int e = 0; e < 4; ++e) bb[e] = (n + e < a.N) ? bf2f(bp[n + e]) : 0.f;
-          }
-#pragma unroll
-          for (int j = 0; j < WT; ++j) {
-            const int tl = j * 16 + (lane & 15);
-            *reinterpret_cast<f32x4_t*>(stg + tl * kStgLd + ((w & 1) * 4 + i) * 16 + q4) =
-                f32x4_t{(acc[i][j][0] + bb[0]) * sc[j], (acc[i][j][1] + bb[1]) * sc[j],
-                        (acc[i][j][2] + bb[2]) * sc[j], (acc[i][j][3] + bb[3]) * sc[j]};
-          }
-        }
-      }
-      __syncthreads();
-      const int c4 = (tid & 31) * 4;                  // row offset within the half
-      const int n = (jb.nb0 + half * 8) * 16 + c4;
-      for (int tl = tid >> 5; tl < NT; tl += 8) {
-        if (jb.t0 + tl >= jb.count) break;
-        const f32x4_t v = *reinterpret_cast<const f32x4_t*>(stg + tl * kStgLd + c4);
-        float* y = ybase + (long long)orow_s[tl] * a.ldy + n;
+        for (int e = 0; e < 4; ++e) v[e] = (v[e] + bb[e]) * sc;
+        float* y = ybase + (long long)row * a.ldy + n;
         if (n + 3 < a.N) {
-          *reinterpret_cast<f32x4_t*>(y) = v;
+          if (a.grp_expert) __builtin_nontemporal_store(v, reinterpret_cast<f32x4_t*>(y));
+          else *reinterpret_cast<f32x4_t*>(y) = v;
         } else {
 #pragma unroll
           for (int e = 0; e < 4; ++e)
             if (n + e < a.N) y[e] = v[e];
         }
       }
-      __syncthreads();                   // the half is read before the next one is written
+      wave_lds_sync();
     }
   }
 }
@@ -366,14 +361,14 @@ MKD_DEV void tile_body(const GemmArgs& a, const TileJob& jb, char* lds) {
 }  // namespace
 
 template <int EPI>
-__global__ void __launch_bounds__(64 * kNW, 2) gemm_tile_kernel(GemmArgs a, int gx) {
+__global__ void __launch_bounds__(64 * kNW, 2) gemm_tile_kernel(GemmArgs a, int gx, int dense_tok) {
   extern __shared__ __attribute__((aligned(16))) char tile_lds[];
   char* lds = tile_lds;
   const int tid = threadIdx.x, lane = tid & 63;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);   // wave-uniform in an SGPR
   // Grid: gx n tiles x work items, linear.  Work items are the token tiles of all
-  // groups in group order (group g owns ceil(count_g / 128) consecutive items); the grid
-  // holds an upper bound (ceil(T*K / 128) + groups) and the block finds its
+  // groups in group order (group g owns ceil(count_g / 160) consecutive items); the grid
+  // holds an upper bound (ceil(T*K / 160) + groups) and the block finds its
   // group by a scan of the device-side group counts.  XCD-aware order: blocks
   // are dealt round-robin to the 8 XCDs by linear id, so each XCD is given a
   // contiguous run of the LIVE logical tiles (n tile fastest, then item): the
@@ -422,13 +417,16 @@ __global__ void __launch_bounds__(64 * kNW, 2) gemm_tile_kernel(GemmArgs a, int 
     const int end = before + x, mid = end - tiles1, beg = mid - tiles0;
     if (mine && item >= beg && item < end) {
       item_s[0] = item < mid ? g0 : g0 + 1;
-      item_s[1] = (item - (item < mid ? beg : mid)) * kTileTok;
+      item_s[1] = item - (item < mid ? beg : mid);
     }
     __syncthreads();
     const int g = __builtin_amdgcn_readfirstlane(item_s[0]);
     if (g < 0) return;                   // past the last live token tile (uniform)
-    jb.t0 = __builtin_amdgcn_readfirstlane(item_s[1]);
-    jb.count = a.grp_count[g];
+    const int k = __builtin_amdgcn_readfirstlane(item_s[1]);
+    const int cnt = a.grp_count[g];
+    const int per = tile_even_rule(cnt, kTileTok);   // the group's equal tiles
+    jb.t0 = k * per;
+    jb.count = min(cnt, jb.t0 + per);
     jb.base = a.grp_offset[g];
     jb.expert = a.grp_expert[g];
     jb.wp += (long long)jb.expert * a.w_group_stride;
@@ -441,20 +439,23 @@ __global__ void __launch_bounds__(64 * kNW, 2) gemm_tile_kernel(GemmArgs a, int 
     const int items = (int)gridDim.x / gx / (a.kgrid > 1 ? a.kgrid : 1);
     const int r = lt / gx;
     jb.kq = r / items;
-    jb.count = a.T;
     jb.base = 0;
-    jb.t0 = (r - jb.kq * items) * kTileTok;
-    if (jb.t0 >= jb.count) return;
+    jb.t0 = (r - jb.kq * items) * dense_tok;
+    jb.count = min(a.T, jb.t0 + dense_tok);
+    if (jb.t0 >= a.T) return;
   }
   jb.nb0 = (lt % gx) * kRB;
   jb.S = a.grp_expert || a.kgrid <= 1 ? a.K / 32 : a.K / 32 / a.kgrid;
   jb.s0 = jb.kq * jb.S;
-  const int live = min(jb.count - jb.t0, kTileTok);
-  if (jb.S & 3) tile_body<EPI, 8, false>(a, jb, lds);
+  const int live = jb.count - jb.t0;
+  if (jb.S & 3) tile_body<EPI, 10, false>(a, jb, lds);
   else if (live <= 32) tile_body<EPI, 2, true>(a, jb, lds);
   else if (live <= 64) tile_body<EPI, 4, true>(a, jb, lds);
   else if (live <= 96) tile_body<EPI, 6, true>(a, jb, lds);
-  else tile_body<EPI, 8, true>(a, jb, lds);
+  else if (live <= 112) tile_body<EPI, 7, true>(a, jb, lds);
+  else if (live <= 128) tile_body<EPI, 8, true>(a, jb, lds);
+  else if (live <= 144) tile_body<EPI, 9, true>(a, jb, lds);
+  else tile_body<EPI, 10, true>(a, jb, lds);
 }
 
 int gemm_tile_lds_bytes() { return kLdsBytes; }
@@ -477,7 +478,7 @@ bool gemm_tile_kgrid_ok(int K, int kgrid) {
 // per slice.  The partials cost T * N * 4 bytes per slice
 // written and read again by the consumer.
 int gemm_tile_kgrid(int N, int K, int T) {
-  static_assert(kTileRows == 256 && kTileTok == 128, "tile_kgrid_rule counts 256 x 2 x 128 tile pairs");
+  static_assert(kTileRows == 256, "tile_kgrid_rule counts 256 x 2 x 128 tile pairs");
   return tile_kgrid_rule(N, K, T, device_cus());
 }
 
@@ -494,22 +495,24 @@ hipError_t gemm_tile_launch(const GemmArgs& a, int epi, int groups_max, long lon
                  a.part_stride < total_rows * a.ldy))
     return hipErrorInvalidValue;
   // work items: every group's token tiles; with total_rows = sum of the group
-  // sizes, sum_g ceil(c_g / 128) <= ceil(total_rows / 128) + groups
-  const long long items = (total_rows + kTileTok - 1) / kTileTok + (a.grp_expert ? groups_max : 0);
+  // sizes, sum_g ceil(c_g / 160) <= ceil(total_rows / 160) + groups.  Dense:
+  // token tiles sized to give every CU one (tile_dense_rule).
   const int gx = (a.N + kTileRows - 1) / kTileRows;
+  const int tok = a.grp_expert ? kTileTok : tile_dense_rule(gx * kg, a.T, device_cus());
+  const long long items = (total_rows + tok - 1) / tok + (a.grp_expert ? groups_max : 0);
   if (items * kg * gx > 0x7fffffff / (64 * kNW)) return hipErrorInvalidValue;
   const dim3 grid((unsigned)(items * kg * gx));
-  // 66.5 KiB of dynamic LDS is above the default launch limit (set per kernel)
+  // 80 KiB of dynamic LDS is above the default launch limit (set per kernel)
   if (epi == EPI_SWIGLU_BF16) {
     if (hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_tile_kernel<EPI_SWIGLU_BF16>),
                                            hipFuncAttributeMaxDynamicSharedMemorySize, kLdsBytes))
       return e;
-    return timed_launch(gemm_tile_kernel<EPI_SWIGLU_BF16>, grid, dim3(64 * kNW), kLdsBytes, s, a, gx);
+    return timed_launch(gemm_tile_kernel<EPI_SWIGLU_BF16>, grid, dim3(64 * kNW), kLdsBytes, s, a, gx, tok);
   }
   if (hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_tile_kernel<EPI_SCALE_F32>),
                                          hipFuncAttributeMaxDynamicSharedMemorySize, kLdsBytes))
     return e;
-  return timed_launch(gemm_tile_kernel<EPI_SCALE_F32>, grid, dim3(64 * kNW), kLdsBytes, s, a, gx);
+  return timed_launch(gemm_tile_kernel<EPI_SCALE_F32>, grid, dim3(64 * kNW), kLdsBytes, s, a, gx, tok);
 }
 
 }  // namespace mkd

@@ -43,6 +43,30 @@ MKD_RULE bool tile_deal_rule(int live, int L, int* lt) {
   return k < q + (xcd < r ? 1 : 0);
 }
 
+// Tokens per tile of a group of `count`: its ceil(count / most) tiles made equal, in
+// whole 16-token columns (`most` a multiple of 16; the last tile may hold fewer).
+MKD_RULE int tile_even_rule(int count, int most) {
+  const int tiles = (count + most - 1) / most;
+  if (tiles <= 1) return most;
+  return ((count + tiles - 1) / tiles + 15) / 16 * 16;
+}
+
+// Tokens per tile of a dense tiled GEMM over T tokens with g tiles per token tile
+// (n tiles x K slices): 128 where that gives every CU a tile, else the smallest
+// multiple of 16 from 64 whose tiles do not outnumber the CUs.  Measured on 256
+// CUs: N 2048, K 4096 at 2048 tokens 56 us with 128-token tiles (128 of them), 40 with
+// 64; N 5120, K 2048 at 512 tokens 32 and 29; but a few tiles more than CUs put two on
+// some (N 5120 at 1024 tokens 46 with 80, 260 tiles), and once the CUs have tiles,
+// smaller ones only re-read the weights more often (N 5120 at 2048 tokens 57 with
+// 128, 65 with 96; at 4096 96, and 135 with 64).
+MKD_RULE int tile_dense_rule(int g, int T, int cus) {
+  if (cus <= 0) cus = 256;
+  int t = 128;
+  if ((long long)((T + t - 1) / t) * g >= cus) return t;
+  while (t > 64 && (long long)((T + t - 17) / (t - 16)) * g <= cus) t -= 16;
+  return t;
+}
+
 // K slices for a dense tiled GEMM (256 x 256 output tiles, 32-wide stages) whose
 // tiles leave CUs idle: the largest of 2, 4, 8 that divides the stage count,
 // keeps at least 16 stages per slice and tiles x slices within the CU count

@@ -91,13 +91,13 @@ def test_moe_prefill_rejects_unsupported(mk, dev):
                        torch.zeros(4, 1, dtype=torch.int32, device=dev))
 
 
-# Group sizes at the edges of the token tiles (128) and of the inner loops (32, 64,
-# 96 and 128 tokens), and k steps (H / 32, I / 32) that leave the four-step loop
+# Group sizes at the edges of the token tiles (160, and the equal parts of larger
+# groups) and of the inner loops (32 .. 160 tokens), and k steps (H / 32, I / 32) that leave the four-step loop
 # after any step.  Same tolerance as above: bf16 h and fp32 sums over K <= 416.
 @pytest.mark.parametrize("H,I", [(32, 32), (64, 96), (96, 160), (128, 224), (288, 64), (416, 128)])
 def test_moe_prefill_group_and_k_edges(mk, dev, H, I):
     from nki_moe_megakernel_amd.common_types import ExpertAffinityScaleMode
-    counts = [0, 1, 31, 32, 33, 63, 64, 65, 95, 96, 97, 127, 128, 129, 160, 257, 0]
+    counts = [0, 1, 31, 32, 33, 64, 65, 96, 97, 112, 113, 127, 128, 129, 144, 145, 160, 161, 321, 0]
     print(f"moe_prefill group edges H={H} I={I}", flush=True)
     E, T = len(counts), sum(counts)
     x, gu, dn, _, _, _, _ = _case(T, E, 1, H, I, False, seed=H + I)
