@@ -71,9 +71,10 @@ MKD_DEV void block_barrier() {
   asm volatile("s_barrier" ::: "memory");
   __builtin_amdgcn_sched_barrier(0);
 }
-// A non-template wrapper (the builtin stays out of template instantiation).
+// (NT: the non-temporal cache policy, bit 1 of the auxiliary operand.)
+template <bool NT>
 MKD_DEV u32x4_t load_frag(__amdgpu_buffer_rsrc_t src, int voff, int soff) {
-  return __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(src, voff, soff, 0));
+  return __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(src, voff, soff, NT ? 2 : 0));
 }
 MKD_DEV void copy_rows_lds(__amdgpu_buffer_rsrc_t src, void* dst, int voff, int soff) {
   __builtin_amdgcn_raw_ptr_buffer_load_lds(src, (__attribute__((address_space(3))) void*)dst, 16, voff,
@@ -95,9 +96,13 @@ struct TileJob {
 };
 
 // The k loop and epilogue for tiles of at most 16 * WT tokens; PAIRS: the k steps
-// are a multiple of 4.  Weight fragments are loaded four k steps ahead, two where
+// are a multiple of 4.  ONCE: the group is this one tile, so no other block reads its
+// weights: they are loaded non-temporal, which leaves the caches to the token rows
+// (moe_prefill at 300 tokens 237 -> 219 us, at 1003 294 -> 270, at 2048 351 -> 344; with
+// several tiles per group it would cost them their shared reads, 2048 tokens in
+// 128-token tiles 347 -> 385).  Weight fragments are loaded four k steps ahead, two where
 // the accumulators leave no registers for more (WT > 8).
-template <int EPI, int WT, bool PAIRS>
+template <int EPI, int WT, bool PAIRS, bool ONCE = false>
 MKD_DEV void tile_body(const GemmArgs& a, const TileJob& jb, char* lds) {
   constexpr int C = (WT + 1) / 2;        // 8-token copies per wave per stage
   constexpr int H0 = (WT + 1) / 2, H1 = WT / 2;   // token tiles of a step's halves
@@ -147,7 +152,7 @@ MKD_DEV void tile_body(const GemmArgs& a, const TileJob& jb, char* lds) {
     const int vo = lane * 16 | (step < S ? 0 : -1);
     issue_fence();
 #pragma unroll
-    for (int i = 0; i < 4; ++i) f[i] = load_frag(wsrc, vo, aoff[i] + step * 1024);
+    for (int i = 0; i < 4; ++i) f[i] = load_frag<ONCE>(wsrc, vo, aoff[i] + step * 1024);
     issue_fence();
   };
   // ---- operand reads: token tile j, step h of the stage in ring slot s % 4 ----
@@ -385,6 +390,7 @@ __global__ void __launch_bounds__(64 * kNW, 2) gemm_tile_kernel(GemmArgs a, int 
   // holds at least `live` blocks, so every tile is taken)
   auto deal = [&](int live, int& lt) { return tile_deal_rule(live, L, &lt); };
   int lt = 0;
+  bool once = false;                     // a group of one tile
 
   TileJob jb;
   jb.wp = a.w;
@@ -427,6 +433,7 @@ __global__ void __launch_bounds__(64 * kNW, 2) gemm_tile_kernel(GemmArgs a, int 
     const int per = tile_even_rule(cnt, kTileTok);   // the group's equal tiles
     jb.t0 = k * per;
     jb.count = min(cnt, jb.t0 + per);
+    once = cnt <= kTileTok;
     jb.base = a.grp_offset[g];
     jb.expert = a.grp_expert[g];
     jb.wp += (long long)jb.expert * a.w_group_stride;
@@ -448,14 +455,23 @@ __global__ void __launch_bounds__(64 * kNW, 2) gemm_tile_kernel(GemmArgs a, int 
   jb.S = a.grp_expert || a.kgrid <= 1 ? a.K / 32 : a.K / 32 / a.kgrid;
   jb.s0 = jb.kq * jb.S;
   const int live = jb.count - jb.t0;
-  if (jb.S & 3) tile_body<EPI, 10, false>(a, jb, lds);
-  else if (live <= 32) tile_body<EPI, 2, true>(a, jb, lds);
-  else if (live <= 64) tile_body<EPI, 4, true>(a, jb, lds);
-  else if (live <= 96) tile_body<EPI, 6, true>(a, jb, lds);
-  else if (live <= 112) tile_body<EPI, 7, true>(a, jb, lds);
-  else if (live <= 128) tile_body<EPI, 8, true>(a, jb, lds);
-  else if (live <= 144) tile_body<EPI, 9, true>(a, jb, lds);
-  else tile_body<EPI, 10, true>(a, jb, lds);
+  if (jb.S & 3) {
+    tile_body<EPI, 10, false>(a, jb, lds);
+  } else if (once) {
+    if (live <= 32) tile_body<EPI, 2, true, true>(a, jb, lds);
+    else if (live <= 64) tile_body<EPI, 4, true, true>(a, jb, lds);
+    else if (live <= 96) tile_body<EPI, 6, true, true>(a, jb, lds);
+    else if (live <= 128) tile_body<EPI, 8, true, true>(a, jb, lds);
+    else tile_body<EPI, 10, true, true>(a, jb, lds);
+  } else {                               // (grouped: 81 .. 160 tokens but for a last tile)
+    if (live <= 32) tile_body<EPI, 2, true>(a, jb, lds);
+    else if (live <= 64) tile_body<EPI, 4, true>(a, jb, lds);
+    else if (live <= 96) tile_body<EPI, 6, true>(a, jb, lds);
+    else if (live <= 112) tile_body<EPI, 7, true>(a, jb, lds);
+    else if (live <= 128) tile_body<EPI, 8, true>(a, jb, lds);
+    else if (live <= 144) tile_body<EPI, 9, true>(a, jb, lds);
+    else tile_body<EPI, 10, true>(a, jb, lds);
+  }
 }
 
 int gemm_tile_lds_bytes() { return kLdsBytes; }
