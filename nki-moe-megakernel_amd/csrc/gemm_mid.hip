@@ -15,6 +15,8 @@
 // so there is no cross-wave reduction; block (row group, kb) writes partial kb
 // of the K split to y + kb * part_stride (bias in partial 0), which the
 // consumer (attention head preparation, post-attention norm) adds in order.
+#include <type_traits>
+#include "coherent.h"
 #include "common.h"
 #include "mkd_internal.h"
 
@@ -203,7 +205,11 @@ int gemm_mid_kgrid(int N, int K, int T, int max_parts) {
 // 17..128 tokens): each block owns 4 * RBW row blocks over the WHOLE K range,
 // looping over K slices of NF fragments -- the slice's activations staged in
 // LDS, the wave's weight fragments streamed -- and writes finished fp32 rows
-// (bias added), so there are no K-split partials to write and read back.  One
+// (bias added), so there are no K-split partials to write and read back.  Bound by
+// HBM (the weights once).  The next slice's loads go out as this one's registers
+// free up and the barriers wait for LDS alone, so weights are always in flight
+// (mkd_lm_head_greedy, N 201088, K 3072: 247 -> 241 us at 32 tokens, 289 -> 279 at 64,
+// 375 -> 364 at 128; N 151936, K 2048: 160 -> 156 at 64).  One
 // 16-row block per launch block instead (the weight-streaming GEMM) reads the
 // activations of every token for every weight fragment through the CU:
 // 4 bytes per weight byte at 64 tokens.
@@ -227,43 +233,54 @@ __global__ void __launch_bounds__(256) gemm_kloop_kernel(GemmArgs a) {
     const int rb = min(blockIdx.x * kMidWaves * RBW + r * kMidWaves + w, NRB - 1);
     wp[r] = a.w + (long long)rb * KB * 512 + lane * 8;
   }
-  for (int sl = 0; sl < nsl; ++sl) {
-    const int kf0 = sl * NF;
-    // the slice's weight fragments, then its activation chunks (L2-resident)
-    u32x4_t wf[RBW][NF];
-#pragma unroll
-    for (int r = 0; r < RBW; ++r)
-#pragma unroll
-      for (int f = 0; f < NF; ++f)
-        wf[r][f] = __builtin_nontemporal_load(reinterpret_cast<const u32x4_t*>(wp[r] + (kf0 + f) * 512));
-    u32x4_t v[PJ];
+  u32x4_t wf[RBW][NF], v[PJ];
+  auto load_w = [&](int r, int f, int sl) {
+    wf[r][f] = __builtin_nontemporal_load(reinterpret_cast<const u32x4_t*>(wp[r] + (sl * NF + f) * 512));
+  };
+  auto load_x = [&](int sl) {
 #pragma unroll
     for (int j = 0; j < PJ; ++j) {
       const int c = threadIdx.x + j * 256;
       const int l = c & 63, f = (c >> 6) % NF, tt = c / (64 * NF);
       const int t = tt * 16 + (l & 15);
       v[j] = ld16(static_cast<const uint16_t*>(a.x) + (long long)(t < a.T ? t : 0) * a.ldx +
-                  (long long)(kf0 + f) * 32 + (l >> 4) * 8);
+                  (long long)(sl * NF + f) * 32 + (l >> 4) * 8);
     }
-    __syncthreads();                               // the previous slice's reads of xs are done
+  };
+  // One slice; MORE: the next slice's activation chunks are loaded once this one's
+  // are in LDS, its weight fragments into each register as its MFMAs have read it.
+  // The chunks go out first: the wait for them leaves the weights in flight.
+  auto slice = [&](int sl, auto more) {
+    constexpr bool MORE = decltype(more)::value;
+    lds_barrier();                                 // the previous slice's reads of xs are done
 #pragma unroll
     for (int j = 0; j < PJ; ++j) {
       const int c = threadIdx.x + j * 256;
       const bool live = (c / (64 * NF)) * 16 + (c & 15) < a.T;
       xs[c] = live ? v[j] : u32x4_t{0u, 0u, 0u, 0u};
     }
-    __syncthreads();
+    if constexpr (MORE) load_x(sl + 1);
+    lds_barrier();
 #pragma unroll
     for (int f = 0; f < NF; ++f) {
       u32x4_t xf[TT];
 #pragma unroll
       for (int tt = 0; tt < TT; ++tt) xf[tt] = xs[(tt * NF + f) * 64 + lane];
 #pragma unroll
-      for (int r = 0; r < RBW; ++r)
+      for (int r = 0; r < RBW; ++r) {
 #pragma unroll
         for (int tt = 0; tt < TT; ++tt) acc[r][tt] = mfma16x16x32(wf[r][f], xf[tt], acc[r][tt]);
+        if constexpr (MORE) load_w(r, f, sl + 1);
+      }
     }
-  }
+  };
+  load_x(0);
+#pragma unroll
+  for (int f = 0; f < NF; ++f)
+#pragma unroll
+    for (int r = 0; r < RBW; ++r) load_w(r, f, 0);
+  for (int sl = 0; sl + 1 < nsl; ++sl) slice(sl, std::true_type{});
+  slice(nsl - 1, std::false_type{});
   float* yb = static_cast<float*>(a.y);
 #pragma unroll
   for (int r = 0; r < RBW; ++r) {
@@ -292,10 +309,12 @@ __global__ void __launch_bounds__(256) gemm_kloop_kernel(GemmArgs a) {
   }
 }
 
-constexpr int kKloopRBW = 2, kKloopNF = 8;
+// Slices of 4 fragments: at 8, the registers of the next slice's loads cost the 128-token
+// form a wave per SIMD (K 3072, N 201088: 418 us a call against 364).
+constexpr int kKloopRBW = 2, kKloopNF = 4;
 
 bool gemm_kloop_supported(int N, int K, int T) {
-  return T >= 17 && T <= 128 && K % (32 * kKloopNF) == 0 && N > 0 &&
+  return T >= 17 && T <= 128 && K % 256 == 0 && N > 0 &&
          (long long)((N + 15) / 16 + kMidWaves * kKloopRBW - 1) / (kMidWaves * kKloopRBW) >= 1024;
 }
 

@@ -897,6 +897,37 @@ def test_lm_head_greedy_many_tokens(mk, dev, B):
             assert int(nxt[b]) == int(nxt_ref[b]), b
 
 
+@pytest.mark.parametrize("B,H,V", [(17, 256, 131072 - 112), (33, 768, 131072 + 16), (65, 256, 131072 + 8),
+                                   (128, 1280, 131072)])
+def test_lm_head_slices_and_row_edges(mk, dev, B, H, V):
+    """Two to ten activation slices (H / 128), the last block's row blocks partly or
+    all past V, one token into a new 16-token tile; fp32 reference of the same product.
+    Products of bf16 values are exact in fp32, so only the order of the H additions and
+    the bf16 rounding of the norm (2^-9 per element, the two sides' norms within one
+    rounding of each other) differ: TOL as in the test above."""
+    from nki_moe_megakernel_amd import packing
+    L = _lib(mk)
+    lib = L.load()
+    print(f"lm_head edges: B={B} H={H} V={V}", flush=True)
+    g = torch.Generator().manual_seed(B + H)
+    x = bf(torch.randn(B, H, generator=g))
+    lnf = bf(1 + 0.1 * torch.randn(H, generator=g))
+    lm = bf(0.05 * torch.randn(V, H, generator=g))
+    packed = packing.pack_out_in(lm.to(dev))
+    logits = torch.full((B + 1, V), 7.0, dtype=torch.float32, device=dev)   # a guard row
+    nxt = torch.empty(B, dtype=torch.int32, device=dev)
+    ws = torch.zeros(lib.mkd_lm_head_workspace_bytes(B, H, V), dtype=torch.uint8, device=dev)
+    xd, lnd = x.to(dev), lnf.to(dev)
+    L.check(lib.mkd_lm_head_greedy(xd.data_ptr(), lnd.data_ptr(), 1e-6, packed.data_ptr(), B, H, V, H, 2,
+                                   logits.data_ptr(), nxt.data_ptr(), ws.data_ptr(), ws.numel(),
+                                   L.stream_ptr(dev)), "lm_head")
+    torch.cuda.synchronize()
+    lg_ref, _ = ref.final_norm_lm_head(x.float(), lnf, lm, 1e-6)
+    assert max_abs_rel(logits[:B], lg_ref) < TOL
+    assert bool((logits[B] == 7.0).all())
+    assert torch.equal(nxt.cpu().long(), logits[:B].argmax(-1).cpu())
+
+
 # ---------------------------------------------------------------- GPT-OSS layer
 def _dequant_mx_torch(codes, scales, fmt, k):
     """Independent dequantiser for the test: element value table x 2^(scale-127)."""
