@@ -390,8 +390,8 @@ int moe_core(const uint16_t* hidden, const void* gate_up, const void* down, cons
     return MKD_OK;
   }
   if (tiled) {
-    // Many tokens per expert: LDS-tiled grouped GEMMs (256 x 256 tiles), one
-    // token tile per 256 tokens of the largest possible group (T).
+    // Many tokens per expert: tiled grouped GEMMs (256 weight rows x up to 160
+    // tokens; each group's tiles are cut on the device).
     {
       GemmArgs a = dense_args(gate_up, hidden, H, 2 * I, H, T, w.hbuf, I);
       a.w_group_stride = (long long)2 * I * H;

@@ -67,10 +67,10 @@ MKD_RULE int tile_dense_rule(int g, int T, int cus) {
   return t;
 }
 
-// K slices for a dense tiled GEMM (256 x 256 output tiles, 32-wide stages) whose
-// tiles leave CUs idle: the largest of 2, 4, 8 that divides the stage count,
-// keeps at least 16 stages per slice and tiles x slices within the CU count
-// (cus <= 0: taken as 256).
+// K slices for a dense tiled GEMM whose output leaves CUs idle, counted in 256 x 256
+// tiles (two blocks of 128 tokens, one pair per CU): the largest of 2, 4, 8 that
+// divides the 32-wide k steps, keeps at least 16 of them per slice and tiles x slices
+// within the CU count (cus <= 0: taken as 256).
 MKD_RULE int tile_kgrid_rule(int N, int K, int T, int cus) {
   if (cus <= 0) cus = 256;
   if (K <= 0 || K % 32 != 0 || N <= 0 || T <= 0) return 1;
