@@ -21,8 +21,9 @@
 // FP8 caches (e4m3 codes, attention_block_tkg.py:133-134, :749-754): a code is
 // exactly a bf16 value, so the scores are those of the stored values with fp32
 // accumulation; the probabilities, which this path keeps in fp32, go to the MFMA
-// as bf16 hi + lo (2^-17 relative).  Each lane reads 32 contiguous bytes of a K row
-// (head elements (l/16) D/4 .. , in the q operand alike).
+// as three bf16 terms that add up to the fp32 value (8 significand bits each).
+// Each lane reads 32 contiguous bytes of a K row (head elements (l/16) D/4 .. , in
+// the q operand alike).
 //
 // A 16-position tile lies in one cache block (block lengths are multiples of 16
 // here; others keep attn_fused_kernel / attn_kvfmt_kernel), so its base address is
@@ -289,7 +290,7 @@ __global__ void __launch_bounds__(64 * kStWaves, FP8 && D == 64 ? 4 : 3) attn_st
 #pragma unroll
         for (int i = 0; i < 4; ++i) o[dt][i] *= al[i];
     }
-    u32x4_t ph, pl;
+    u32x4_t ph, pm, pl;                       // p = ph (+ pm + pl for FP8: exact)
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
       float p[4];
@@ -301,8 +302,13 @@ __global__ void __launch_bounds__(64 * kStWaves, FP8 && D == 64 ? 4 : 3) attn_st
       ph[2 * u] = pack2bf(p[0], p[1]);
       ph[2 * u + 1] = pack2bf(p[2], p[3]);
       if constexpr (FP8) {
-        pl[2 * u] = pack2bf(p[0] - bf_lo(ph[2 * u]), p[1] - bf_hi(ph[2 * u]));
-        pl[2 * u + 1] = pack2bf(p[2] - bf_lo(ph[2 * u + 1]), p[3] - bf_hi(ph[2 * u + 1]));
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+          const int j = 2 * u + k;
+          const float r0 = p[2 * k] - bf_lo(ph[j]), r1 = p[2 * k + 1] - bf_hi(ph[j]);
+          pm[j] = pack2bf(r0, r1);
+          pl[j] = pack2bf(r0 - bf_lo(pm[j]), r1 - bf_hi(pm[j]));
+        }
       }
     }
     // ---- P . V ----
@@ -322,33 +328,32 @@ __global__ void __launch_bounds__(64 * kStWaves, FP8 && D == 64 ? 4 : 3) attn_st
         }
     }
     if constexpr (FP8) {
-      // four head elements (one dword of each row) at a time
+      // two head elements (half a dword of each row) at a time
 #pragma unroll
-      for (int e = 0; e < VD; ++e) {
-        float x[2][4][4];
+      for (int e = 0; e < 2 * VD; ++e) {
+        float x[2][4][2];
 #pragma unroll
         for (int u = 0; u < 2; ++u)
 #pragma unroll
           for (int j = 0; j < 4; ++j) {
-            const f32x2_t lo = cvt2_fp8_lo(vr[u][j][e]), hi = cvt2_fp8_hi(vr[u][j][e]);
-            x[u][j][0] = lo[0];
-            x[u][j][1] = lo[1];
-            x[u][j][2] = hi[0];
-            x[u][j][3] = hi[1];
+            const f32x2_t v = (e & 1) ? cvt2_fp8_hi(vr[u][j][e >> 1]) : cvt2_fp8_lo(vr[u][j][e >> 1]);
+            x[u][j][0] = v[0];
+            x[u][j][1] = v[1];
             if (edge) {
               const int t = p0 + 16 * u + 4 * q4 + j;
               if (t >= n && t < total) {
 #pragma unroll
-                for (int k = 0; k < 4; ++k) x[u][j][k] = bf2f(vn_s[t - n][col * NDT + 4 * e + k]);
+                for (int k = 0; k < 2; ++k) x[u][j][k] = bf2f(vn_s[t - n][col * NDT + 2 * e + k]);
               }
             }
           }
 #pragma unroll
-        for (int k = 0; k < 4; ++k) {
+        for (int k = 0; k < 2; ++k) {
           const u32x4_t bop = {pack2bf(x[0][0][k], x[0][1][k]), pack2bf(x[0][2][k], x[0][3][k]),
                                pack2bf(x[1][0][k], x[1][1][k]), pack2bf(x[1][2][k], x[1][3][k])};
-          o[4 * e + k] = mfma16x16x32(ph, bop, o[4 * e + k]);
-          o[4 * e + k] = mfma16x16x32(pl, bop, o[4 * e + k]);
+          o[2 * e + k] = mfma16x16x32(ph, bop, o[2 * e + k]);
+          o[2 * e + k] = mfma16x16x32(pm, bop, o[2 * e + k]);
+          o[2 * e + k] = mfma16x16x32(pl, bop, o[2 * e + k]);
         }
       }
     } else {

@@ -3,10 +3,12 @@ oracle, at the edges of its steps (32 positions), chunks (64 .. 512) and cache b
 block lengths it leaves to the general kernels.
 
 Tolerance: max-abs-rel 2e-2, the bf16 bound of the other attention tests (probabilities rounded to
-bf16, or hi + lo for FP8, and a bf16 output).  The same logical cache through block lengths 16 / 32 /
+bf16, kept in fp32 for FP8, and a bf16 output).  The same logical cache through block lengths 16 / 32 /
 64 (streaming) and 24 (general kernels) differs only by the two kernels' summation orders and their
 bf16 roundings of the probabilities: held to 1e-2.
 """
+import math
+
 import pytest
 import torch
 
@@ -78,6 +80,30 @@ def test_fp8_stream_matches_oracle(mk, dev, blk, B, nq, nkv, d, NT, P):
     print(f"fp8 stream blk={blk} B={B} nq={nq} nkv={nkv} d={d} NT={NT} P={P}", flush=True)
     out, want = _run(mk, dev, True, blk, B, nq, nkv, d, NT, P)
     assert max_abs_rel(out, want) < 2e-2
+
+
+@pytest.mark.parametrize("d,a,b", [(128, 11, 15), (64, 12, 13), (64, 8, 9)])
+def test_fp8_probabilities_keep_fp32(mk, dev, d, a, b):
+    """Two positions of probability 1 and r = a / b (unnormalised; scores ln(b / a) and 0) with values
+    -16 a and 16 b, and a new token of zeros: the head's output is 16 b (r - a / b) / (1 + 2 r), which
+    shows r's own error.  In fp32 that is expf's 2^-23 r and 2^-24 ln(b / a) r of the scale, and the sum
+    of terms up to 16 a rounds three times by at most 2^-24 of it.  (r as two bf16 terms: 2^-18, 6 to 12
+    times the bound.)"""
+    nq, S = 4, 16
+    X, W = torch.zeros(1, 1, 128), torch.zeros(128, d * (nq + 2))
+    X[..., 0] = 1.0
+    W[0, 0:nq * d:d] = 1.0                       # q = e0 for every head; k = v = 0
+    K, V = torch.zeros(1, S, d), torch.zeros(1, S, d)
+    K[0, 1, 0] = 1.0
+    V[0, 0], V[0, 1] = 16.0 * b, -16.0 * a
+    K, V = K.to(torch.float8_e4m3fn), V.to(torch.float8_e4m3fn)
+    ones, one = torch.ones(d // 2, 1, 1), torch.ones(1, 1)
+    out, _, _ = _call(mk, dev, bf(X), bf(W), None, None, None, ones, 0 * ones, K.to(dev), V.to(dev),
+                      torch.ones(3, 1, nq, 1, dtype=torch.uint8), None, torch.tensor([[-1]], dtype=torch.int32),
+                      None, False, one, one, math.log(b / a))
+    r = a / b
+    bound = (16 * b * r * (2.0 ** -23 + 2.0 ** -24 * math.log(b / a)) + 3 * 2.0 ** -24 * 16 * a) / (1 + 2 * r)
+    assert out.float().abs().max().item() <= bound, (out.float().abs().max().item(), bound)
 
 
 # >= 1024 blocks of 256 positions: the streaming kernel; from 2048 blocks of 512: its larger chunk
