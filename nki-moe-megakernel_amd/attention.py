@@ -164,6 +164,8 @@ def attention_block_tkg(
         raise ValueError("cos and sin must be given together")
     if cos is not None and tuple(cos.shape) != (d // 2, B, S_tkg):
         raise ValueError(f"cos shape mismatch: expected ({d // 2}, {B}, {S_tkg}), got {tuple(cos.shape)}")
+    if sin is not None and tuple(sin.shape) != (d // 2, B, S_tkg):
+        raise ValueError(f"sin shape mismatch: expected ({d // 2}, {B}, {S_tkg}), got {tuple(sin.shape)}")
     if update_cache and kv_cache_update_idx is None:
         raise ValueError("update_cache=True needs kv_cache_update_idx")
     if X.dtype != torch.bfloat16:

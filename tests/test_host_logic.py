@@ -54,3 +54,29 @@ def test_prefill_rejects_bad_requests_before_any_gpu_call(mk):
     with pytest.raises(ValueError, match="embedding"):
         _prefill(SimpleNamespace(**{**m.__dict__, "lm_head_packed": None}), ids, 0, 0, 128, 8, 8, 2,
                  lambda p: (None, None))
+
+
+def _attention_call(mk, **kw):
+    """attention_block_tkg on CPU tensors: B 4, H 128, four query heads and one kv head of 64, 31
+    cached positions in a cache of 32; `kw` replaces arguments."""
+    B, d, nq, none = 4, 64, 4, mk.QuantizationType.NONE
+    a = dict(cos=torch.ones(d // 2, B, 1), sin=torch.zeros(d // 2, B, 1),
+             kv_cache_update_idx=torch.zeros(B, 1, dtype=torch.int32))
+    a.update(kw)
+    zeros = lambda *s: torch.zeros(*s, dtype=torch.bfloat16)
+    return mk.attention_block_tkg(
+        zeros(B, 1, 128), None, False, 1e-6, None, zeros(128, d * (nq + 2)), None, none, None, None, False, 1e-6,
+        None, None, a["cos"], a["sin"], True, False, 1e-6, None, None, False, None, zeros(B, 32, d),
+        zeros(B, 32, d), torch.ones(32, B, nq, 1, dtype=torch.uint8), None, True, a["kv_cache_update_idx"], None,
+        None, none, None, None, False, False)
+
+
+@pytest.mark.parametrize("shape", [(32, 1, 1), (16, 4, 1), (32, 4, 2), (32, 8, 1), (32, 4), (128,)])
+def test_attention_refuses_rope_tables_of_another_shape(mk, monkeypatch, shape):
+    """Both tables are indexed over [d/2, B, S_tkg] by their strides, so either of another
+    shape is refused before any kernel (a shorter one would be read past its end)."""
+    from nki_moe_megakernel_amd import _lib as L
+    monkeypatch.setattr(L, "require_gpu", lambda *t: None)
+    for name in ("cos", "sin"):
+        with pytest.raises(ValueError, match=f"{name} shape mismatch"):
+            _attention_call(mk, **{name: torch.zeros(shape)})
