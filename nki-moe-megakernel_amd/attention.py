@@ -168,6 +168,8 @@ def attention_block_tkg(
         raise ValueError(f"sin shape mismatch: expected ({d // 2}, {B}, {S_tkg}), got {tuple(sin.shape)}")
     if update_cache and kv_cache_update_idx is None:
         raise ValueError("update_cache=True needs kv_cache_update_idx")
+    if update_cache and kv_cache_update_idx.numel() < B:   # the kernels read one entry per sequence
+        raise ValueError(f"kv_cache_update_idx must be [B={B}, 1], got {tuple(kv_cache_update_idx.shape)}")
     if X.dtype != torch.bfloat16:
         raise ValueError("X must be bfloat16")
     fp8_types = (torch.float8_e4m3fn, torch.uint8)

@@ -80,3 +80,13 @@ def test_attention_refuses_rope_tables_of_another_shape(mk, monkeypatch, shape):
     for name in ("cos", "sin"):
         with pytest.raises(ValueError, match=f"{name} shape mismatch"):
             _attention_call(mk, **{name: torch.zeros(shape)})
+
+
+@pytest.mark.parametrize("dtype", [torch.int32, torch.int64])
+def test_attention_refuses_too_few_write_positions(mk, monkeypatch, dtype):
+    """One write position per sequence is read; fewer are refused before any kernel."""
+    from nki_moe_megakernel_amd import _lib as L
+    monkeypatch.setattr(L, "require_gpu", lambda *t: None)
+    for shape in ((3, 1), (1,), (0, 1)):
+        with pytest.raises(ValueError, match="kv_cache_update_idx must be"):
+            _attention_call(mk, kv_cache_update_idx=torch.zeros(shape, dtype=dtype))
