@@ -10,6 +10,7 @@ import math
 from typing import Optional
 
 import torch
+from torch.autograd import forward_ad
 
 from . import _lib as L
 from . import packing
@@ -19,6 +20,17 @@ from .common_types import (ActFnType, ExpertAffinityScaleMode, RouterActFnType,
 
 def _ws(nbytes: int, device) -> torch.Tensor:
     return torch.empty(max(nbytes, 256), dtype=torch.uint8, device=device)
+
+
+def _disjoint(tensors) -> bool:
+    """No two of the tensors share memory: storages of their own, or extents apart in a common one."""
+    if len({t.untyped_storage().data_ptr() for t in tensors}) == len(tensors):
+        return True
+    ends = [(t.data_ptr(), t.data_ptr() + t.element_size() * (1 + sum((n - 1) * st for n, st in
+                                                                      zip(t.shape, t.stride()))))
+            for t in tensors if t.numel()]
+    ends.sort()
+    return all(a[1] <= b[0] for a, b in zip(ends, ends[1:]))
 
 
 def router_topk(x: torch.Tensor, w: torch.Tensor, w_bias: Optional[torch.Tensor],
@@ -75,10 +87,17 @@ def router_topk(x: torch.Tensor, w: torch.Tensor, w_bias: Optional[torch.Tensor]
     if xt.dtype not in (torch.float32, torch.bfloat16):
         raise ValueError("x must be bfloat16 or float32")
     dev = x.device
-    # the kernels write the caller's tensors where their layout is the kernels' own (no copies after)
+    bias = w_bias.reshape(-1).to(torch.bfloat16).contiguous() if w_bias is not None else None
+    # The kernels write the caller's tensors where nothing tells them from copy_ afterwards: their
+    # layout is the kernels' own, no memory is shared with an input or another output (the copies'
+    # order would count), autograd does not refuse or record the write.
+    plain = (forward_ad._current_level < 0 and
+             _disjoint([router_logits, expert_affinities, expert_index, xt] + ([bias] if bias is not None else [])))
+
     def direct(t, shape, dtype, wanted=True):
-        if (wanted and t.dtype == dtype and tuple(t.shape) == shape and t.is_contiguous()
-                and t.device == dev and t.data_ptr() % 16 == 0):
+        if (wanted and plain and t.dtype == dtype and tuple(t.shape) == shape and t.is_contiguous()
+                and t.device == dev and t.data_ptr() % 16 == 0 and not t.requires_grad and not t.is_neg()
+                and (not t.is_inference() or torch.is_inference_mode_enabled())):
             return t
         return torch.empty(shape, dtype=dtype, device=dev)
     logits = direct(router_logits, (T, E), torch.float32)
@@ -92,23 +111,23 @@ def router_topk(x: torch.Tensor, w: torch.Tensor, w_bias: Optional[torch.Tensor]
         mode |= L.ROUTER_PRE_NORM
     if norm_topk_prob:
         mode |= L.ROUTER_NORM_TOPK
-    bias = w_bias.reshape(-1).to(torch.bfloat16).contiguous() if w_bias is not None else None
     lib = L.load()
     ws = _ws(lib.mkd_router_workspace_bytes(min(T, 4096), H, E), dev)
+    x_p, logits_p, aff_p, idx_p = xt.data_ptr(), logits.data_ptr(), aff.data_ptr(), idx.data_ptr()
     for t0 in range(0, T, 4096):     # one call per 4096 tokens (the library's bound)
-        t1 = min(T, t0 + 4096)
-        rc = lib.mkd_router_topk(xt[t0:t1].data_ptr(), xdt, t1 - t0, H, wp.data_ptr(), E,
-                                 L.ptr(bias), logits[t0:t1].data_ptr(), aff[t0:t1].data_ptr(),
-                                 idx[t0:t1].data_ptr(), topk[t0:t1].data_ptr() if topk is not None else None,
-                                 k, mode,
+        rc = lib.mkd_router_topk(x_p + t0 * H * xt.element_size(), xdt, min(T - t0, 4096), H, wp.data_ptr(), E,
+                                 L.ptr(bias), logits_p + 4 * t0 * E, aff_p + 4 * t0 * E, idx_p + 4 * t0 * k,
+                                 topk.data_ptr() if topk is not None else None, k, mode,   # (T <= 128)
                                  ws.data_ptr(), ws.numel(), L.stream_ptr(dev))
         L.check(rc, "router_topk")
-    if logits is not router_logits:
-        router_logits.copy_(logits)
-    if aff is not expert_affinities:
-        expert_affinities.copy_(aff)
-    if idx is not expert_index and not skip_store_expert_index:
-        expert_index.copy_(idx)
+    written = []                     # through their pointers
+    for t, new, wanted in ((router_logits, logits, True), (expert_affinities, aff, True),
+                           (expert_index, idx, not skip_store_expert_index)):
+        if new is t:
+            written.append(t)
+        elif wanted:
+            t.copy_(new)
+    torch.autograd.graph.increment_version(written)
     out = [router_logits, expert_index, expert_affinities]
     if return_eager_affi:
         out.append(topk)

@@ -190,3 +190,61 @@ def test_router_writes_callers_tensors(mk, dev):
              torch.empty(T, k, dtype=torch.int64, device=dev))
     for p, q in zip(a, b):
         assert torch.equal(p, q.to(p.dtype))
+
+
+def test_router_outputs_behave_like_copies(mk, dev):
+    """Writing in place keeps what copy_ did: version counters move, a leaf that requires grad is refused,
+    an output that shares memory with another output or the input gets the later one's values."""
+    g = torch.Generator().manual_seed(5)
+    T, H, E, k = 16, 128, 128, 4
+    x, w = torch.randn(T, H, generator=g).to(dev), bf(torch.randn(H, E, generator=g)).float().to(dev)
+
+    def call(x, lg, af, ix):
+        mk.router_topk(x, w, None, lg, af, ix, mk.RouterActFnType.SOFTMAX, k, 1, 0, True, True)
+        return lg, af, ix
+
+    def outs():
+        return (torch.empty(T, E, device=dev), torch.empty(T, E, device=dev),
+                torch.empty(T, k, dtype=torch.int32, device=dev))
+    want = call(x, *outs())
+    fresh = outs()
+    before = [t._version for t in fresh]
+    call(x, *fresh)
+    assert all(t._version > v for t, v in zip(fresh, before))
+    for i in range(2):
+        o = list(outs())
+        o[i].requires_grad_(True)
+        with pytest.raises(RuntimeError, match="leaf Variable that requires grad"):
+            call(x, *o)
+    lg, _, ix = outs()
+    call(x, lg, lg, ix)                                          # affinities are stored last
+    assert torch.equal(lg, want[1]) and torch.equal(ix, want[2])
+    xi = x.clone()                                               # logits over the input
+    _, af, ix = outs()
+    call(xi, xi, af, ix)
+    assert torch.equal(xi, want[0]) and torch.equal(af, want[1]) and torch.equal(ix, want[2])
+    both = torch.empty(2 * T * E, device=dev)                    # parts of one buffer, apart and overlapping
+    got = call(x, both[:T * E].view(T, E), both[T * E:].view(T, E), ix)
+    for a, b in zip(got, want):
+        assert torch.equal(a, b)
+    call(x, both[E:E + T * E].view(T, E), both[:T * E].view(T, E), ix)
+    assert torch.equal(both[:T * E].view(T, E), want[1]) and torch.equal(both[T * E:T * E + E], want[0][-1])
+
+
+def test_router_chunks_land_in_their_rows(mk, dev):
+    """Above 4096 tokens the operator makes a call per 4096: the last call's rows (odd counts, into rows
+    of outputs with a guard after them) equal those of the same tokens alone, a call of the same form."""
+    g = torch.Generator().manual_seed(6)
+    T, H, E, k = 4096 + 133, 128, 24, 3
+    x, w = bf(torch.randn(T, H, generator=g)).to(dev), bf(torch.randn(H, E, generator=g)).to(dev)
+
+    def call(x):
+        n = x.shape[0]
+        lg, af = torch.full((n + 1, E), 7.0, device=dev), torch.full((n + 1, E), 7.0, device=dev)
+        ix = torch.full((n + 1, k), 7, dtype=torch.int32, device=dev)
+        mk.router_topk(x, w, None, lg[:n], af[:n], ix[:n], mk.RouterActFnType.SOFTMAX, k, 1, 0, True, True)
+        assert all(bool((t[n] == 7).all()) for t in (lg, af, ix))
+        return lg[:n], af[:n], ix[:n]
+    whole, first, last = call(x), call(x[:4096]), call(x[4096:])
+    for t, a, b in zip(whole, first, last):
+        assert torch.equal(t[:4096], a) and torch.equal(t[4096:], b)

@@ -90,3 +90,11 @@ def test_attention_refuses_too_few_write_positions(mk, monkeypatch, dtype):
     for shape in ((3, 1), (1,), (0, 1)):
         with pytest.raises(ValueError, match="kv_cache_update_idx must be"):
             _attention_call(mk, kv_cache_update_idx=torch.zeros(shape, dtype=dtype))
+
+
+def test_disjoint_knows_shared_memory(mk):
+    from nki_moe_megakernel_amd.moe import _disjoint
+    a, b = torch.zeros(8, 4), torch.zeros(8, 4)
+    assert _disjoint([a, b]) and _disjoint([a[:4], a[4:], b]) and _disjoint([a[4:], a[:4]])
+    assert not _disjoint([a, a]) and not _disjoint([a[:5], a[4:]]) and not _disjoint([a[:, :2], a[:, 2:]])
+    assert not _disjoint([b, a.t(), a[7:]]) and _disjoint([a[:0], a, b])
