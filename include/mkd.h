@@ -190,7 +190,7 @@ typedef struct {
   const void* down_packed;     /* E x packed [H, I]              */
   const float* expert_affinities; /* [T, E] or NULL               */
   const float* slot_weights;   /* [T*K] or NULL (overrides gather) */
-  const int* expert_index;     /* [T, K]                         */
+  const int* expert_index;     /* [T, K], each token's distinct; an id outside [0, E) adds nothing */
   const void* gate_up_bias;    /* [E, 2, I] bf16 or NULL         */
   const void* down_bias;       /* [E, H] bf16 or NULL            */
   const void* residual;        /* [T, H] bf16 or NULL            */

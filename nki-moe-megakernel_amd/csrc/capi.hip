@@ -343,7 +343,7 @@ int moe_core(const uint16_t* hidden, const void* gate_up, const void* down, cons
       prof_end(ps, s);
     }
     if (do_finalize)
-      MKD_TRY(moe_finalize_launch(w.ybuf, T, K, H, resid, out, out_f32, s), "moe finalize");
+      MKD_TRY(moe_finalize_launch(w.ybuf, T, K, H, idx, E, resid, out, out_f32, s), "moe finalize");
     return MKD_OK;
   }
   if (wfmt) {
@@ -386,7 +386,7 @@ int moe_core(const uint16_t* hidden, const void* gate_up, const void* down, cons
       prof_end(ps, s);
     }
     if (do_finalize)
-      MKD_TRY(moe_finalize_launch(w.ybuf, T, K, H, resid, out, out_f32, s), "moe finalize");
+      MKD_TRY(moe_finalize_launch(w.ybuf, T, K, H, idx, E, resid, out, out_f32, s), "moe finalize");
     return MKD_OK;
   }
   if (tiled) {
@@ -416,7 +416,7 @@ int moe_core(const uint16_t* hidden, const void* gate_up, const void* down, cons
       prof_end(ps, s);
     }
     if (do_finalize)
-      MKD_TRY(moe_finalize_launch(w.ybuf, T, K, H, resid, out, out_f32, s), "moe finalize");
+      MKD_TRY(moe_finalize_launch(w.ybuf, T, K, H, idx, E, resid, out, out_f32, s), "moe finalize");
     return MKD_OK;
   }
   // Routed experts see few tokens each (T*K/E on average), so one 16-token
@@ -449,7 +449,7 @@ int moe_core(const uint16_t* hidden, const void* gate_up, const void* down, cons
     MKD_TRY(moe_fused_launch(f, gmax, s), "moe router select + gate_up + down");
     prof_end(ps, s);
     if (do_finalize)
-      MKD_TRY(moe_finalize_launch(w.ybuf, T, K, H, resid, out, out_f32, s), "moe finalize");
+      MKD_TRY(moe_finalize_launch(w.ybuf, T, K, H, idx, E, resid, out, out_f32, s), "moe finalize");
     return MKD_OK;
   }
   {  // gate/up + activation
@@ -481,7 +481,7 @@ int moe_core(const uint16_t* hidden, const void* gate_up, const void* down, cons
     prof_end(ps, s);
   }
   if (do_finalize)
-    MKD_TRY(moe_finalize_launch(w.ybuf, T, K, H, resid, out, out_f32, s), "moe finalize");
+    MKD_TRY(moe_finalize_launch(w.ybuf, T, K, H, idx, E, resid, out, out_f32, s), "moe finalize");
   return MKD_OK;
 }
 

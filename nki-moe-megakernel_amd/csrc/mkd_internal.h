@@ -557,8 +557,9 @@ struct MoeBegin {
 hipError_t moe_route_launch(const int* idx, int T, int K, int E, int* n_groups, int* grp_expert,
                             int* grp_count, int* grp_offset, int* pair_token, int* pair_slot,
                             hipStream_t s, int* chunk_off = nullptr, const MoeBegin* begin = nullptr);
-hipError_t moe_finalize_launch(const float* ybuf, int T, int K, int H, const uint16_t* resid,
-                               uint16_t* out, float* out_f32, hipStream_t s);
+// (idx [T, K]: slots of an expert id outside [0, E) contribute nothing; null: none)
+hipError_t moe_finalize_launch(const float* ybuf, int T, int K, int H, const int* idx, int E,
+                               const uint16_t* resid, uint16_t* out, float* out_f32, hipStream_t s);
 
 // misc.hip
 hipError_t attn_operands_launch(const mkd_attention_operands& o, hipStream_t s);

@@ -14,8 +14,8 @@
 // moe_route: single block of 1024 threads; counting sort of the T*K (token, k)
 //   slots by expert into compact groups (live experts in ascending id order;
 //   the slots within a group in any order -- every consumer indexes by slot).
-// moe_finalize: out[t] = bf16(sum_k y[t*K + k]) (fp32 sum in k order), then the
-//   bf16 residual add.
+// moe_finalize: out[t] = bf16(sum_k y[t*K + k]) (fp32 sum in k order, over the
+//   slots of existing experts), then the bf16 residual add.
 #include "common.h"
 #include "mkd_internal.h"
 #include "mx_codec.h"
@@ -242,10 +242,13 @@ moe_route_scatter_kernel(const int* __restrict__ idx, int TK, int K, int E, int 
 
 // ---------------------------------------------------------------------------
 // Eight expert rows' loads are in flight before the first is added (8192 tokens x 8
-// rows of 2048: 117 us one row at a time).
+// rows of 2048: 117 us one row at a time).  A slot whose expert id names no expert
+// (idx, null: every slot is live) was routed nowhere: its row holds whatever the
+// workspace held, and is not added.
 __global__ void __launch_bounds__(256)
-moe_finalize_kernel(const float* __restrict__ ybuf, int K, int H, const uint16_t* __restrict__ resid,
-                    uint16_t* __restrict__ out, float* __restrict__ out_f32) {
+moe_finalize_kernel(const float* __restrict__ ybuf, int K, int H, const int* __restrict__ idx, int E,
+                    const uint16_t* __restrict__ resid, uint16_t* __restrict__ out,
+                    float* __restrict__ out_f32) {
   const int t = blockIdx.y;
   const int i = (blockIdx.x * blockDim.x + threadIdx.x) * 4;
   if (i >= H) return;
@@ -258,7 +261,7 @@ moe_finalize_kernel(const float* __restrict__ ybuf, int K, int H, const uint16_t
     for (int k = 0; k < 8; ++k) y[k] = *reinterpret_cast<const f32x4_t*>(y0 + (long long)min(k0 + k, K - 1) * H);
 #pragma unroll
     for (int k = 0; k < 8; ++k)
-      if (k0 + k < K) s += y[k];
+      if (k0 + k < K && (!idx || (unsigned)idx[(long long)t * K + k0 + k] < (unsigned)E)) s += y[k];
   }
   if (out_f32) *reinterpret_cast<f32x4_t*>(out_f32 + o0) = s;
   if (out) {
@@ -478,11 +481,11 @@ hipError_t moe_route_launch(const int* idx, int T, int K, int E, int* n_groups, 
   return hipGetLastError();
 }
 
-hipError_t moe_finalize_launch(const float* ybuf, int T, int K, int H, const uint16_t* resid,
-                               uint16_t* out, float* out_f32, hipStream_t s) {
+hipError_t moe_finalize_launch(const float* ybuf, int T, int K, int H, const int* idx, int E,
+                               const uint16_t* resid, uint16_t* out, float* out_f32, hipStream_t s) {
   if (H % 4 != 0) return hipErrorInvalidValue;
   hipLaunchKernelGGL(moe_finalize_kernel, dim3((H / 4 + 255) / 256, T), dim3(256), 0, s, ybuf, K,
-                     H, resid, out, out_f32);
+                     H, idx, E, resid, out, out_f32);
   return hipGetLastError();
 }
 

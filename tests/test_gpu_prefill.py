@@ -110,3 +110,48 @@ def test_moe_prefill_group_and_k_edges(mk, dev, H, I):
     torch.cuda.synchronize()
     y_ref = ref.moe_tkg(x, gu, dn, aff, idx.long(), None, None, "post", "silu")
     assert max_abs_rel(out, y_ref) < TOL
+
+
+@pytest.mark.parametrize("form,T,K", [("bf16", 5, 3), ("bf16", 128, 8), ("prefill", 300, 3), ("fp8", 33, 2),
+                                      ("mxfp4", 16, 4)])
+def test_slots_without_an_expert_add_nothing(mk, dev, monkeypatch, form, T, K):
+    """Expert ids outside [0, E) over a workspace full of NaN: such a slot's row is written by no expert
+    GEMM, so the result is bit for bit that of the slot at an expert of affinity 0 (one per slot: a token
+    names an expert once); a token whose every slot is such gives zeros."""
+    from nki_moe_megakernel_amd import mx
+    from nki_moe_megakernel_amd.common_types import ExpertAffinityScaleMode
+    E, H, I = 16 + K, 512, 128
+    x, gu, dn, _, _, _, _ = _case(T, E, K, H, I, False, seed=T + K)
+    g = torch.Generator().manual_seed(K)
+    bad = torch.rand(T, K, generator=g) < 0.3
+    bad[T // 2] = True
+    idx = torch.stack([torch.randperm(16, generator=g)[:K] for _ in range(T)]).to(torch.int32)
+    aff = torch.zeros(T, E)                                      # the last K experts: 0
+    aff[:, :16] = torch.rand(T, 16, generator=g) + 0.5
+    ids = torch.where(bad, torch.tensor([-1, E, 2 ** 31 - 1, -2 ** 31])[torch.randint(0, 4, (T, K), generator=g)],
+                      idx.long()).to(torch.int32)
+    kw = {}
+    gu, dn = gu.to(dev), dn.to(dev)
+    if form == "fp8":
+        gu, dn = (8 * gu.float()).to(torch.float8_e4m3fn), (8 * dn.float()).to(torch.float8_e4m3fn)
+        kw = dict(expert_gate_up_weights_scale=torch.full((E, 2, I), 0.125, device=dev),
+                  expert_down_weights_scale=torch.full((E, H), 0.125, device=dev))
+    elif form == "mxfp4":
+        gu, gs, dn, ds = mx.quantize_experts_mx(gu, dn, 2)
+        kw = dict(expert_gate_up_weights_scale=gs, expert_down_weights_scale=ds)
+
+    def call(ids):
+        kw["expert_affinities_scaling_mode"] = ExpertAffinityScaleMode.POST_SCALE
+        a = (x.to(dev), gu, dn, aff.to(dev), ids.to(dev))
+        return mk.moe_prefill(*a, **kw) if form == "prefill" else mk.moe_tkg(*a, False, **kw)
+    want = call(torch.where(bad, torch.arange(E - K, E, dtype=torch.int32), idx))
+    empty = torch.empty
+
+    def poisoned(*a, **k):
+        t = empty(*a, **k)
+        return t.fill_(255) if t.dtype == torch.uint8 else t
+    monkeypatch.setattr(torch, "empty", poisoned)
+    got = call(ids)
+    torch.cuda.synchronize()
+    assert torch.equal(got, want)
+    assert not got[T // 2].any() and bool(got.any())
