@@ -208,13 +208,15 @@ int gemm_mid_kgrid(int N, int K, int T, int max_parts) {
 // (bias added), so there are no K-split partials to write and read back.  Bound by
 // HBM (the weights once).  The next slice's loads go out as this one's registers
 // free up and the barriers wait for LDS alone, so weights are always in flight
-// (mkd_lm_head_greedy, N 201088, K 3072: 247 -> 241 us at 32 tokens, 289 -> 279 at 64,
-// 375 -> 364 at 128; N 151936, K 2048: 160 -> 156 at 64).  One
+// (mkd_lm_head_greedy, N 201088, K 3072: 247 -> 241 us at 32 tokens, 290 -> 280 at 64,
+// 308 -> 295 at 65, 376 -> 353 at 128; N 151936, K 2048: 160 -> 153 at 64, 207 -> 192 at 128).
+// The 65 .. 128-token form is held to two waves per SIMD: the compiler otherwise takes
+// 260 registers for it, one wave (N 201088, K 3072 at 65 tokens 316 us, at 128 364).  One
 // 16-row block per launch block instead (the weight-streaming GEMM) reads the
 // activations of every token for every weight fragment through the CU:
 // 4 bytes per weight byte at 64 tokens.
 template <int TT, int RBW, int NF>
-__global__ void __launch_bounds__(256) gemm_kloop_kernel(GemmArgs a) {
+__global__ void __launch_bounds__(256, TT == 8 ? 2 : 1) gemm_kloop_kernel(GemmArgs a) {
   extern __shared__ __attribute__((aligned(16))) u32x4_t xs[];    // [TT][NF][64]
   const int lane = threadIdx.x & 63;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -309,8 +311,9 @@ __global__ void __launch_bounds__(256) gemm_kloop_kernel(GemmArgs a) {
   }
 }
 
-// Slices of 4 fragments: at 8, the registers of the next slice's loads cost the 128-token
-// form a wave per SIMD (K 3072, N 201088: 418 us a call against 364).
+// Slices of 4 fragments: at 8, the registers of the next slice's loads cost every form a wave
+// per SIMD (up to 32 and 64 tokens 4 and 3 waves at 4, 3 and 2 at 8), and the 128-token form
+// needs 328 (K 3072, N 201088 at 128 tokens 418 us a call).
 constexpr int kKloopRBW = 2, kKloopNF = 4;
 
 bool gemm_kloop_supported(int N, int K, int T) {
