@@ -96,7 +96,7 @@ __global__ void mx_quantize_e2m1_kernel(const void* __restrict__ x, int rows, in
   for (int j = 0; j < 4; ++j) {
     uint32_t d = 0;
 #pragma unroll
-    for (int h = 0; h < 8; ++h) d |= mx_encode<MX_E2M1>(ldexpf(v[8 * j + h], sh)) << (4 * h);
+    for (int h = 0; h < 8; ++h) d |= mx_encode_e2m1(ldexpf(v[8 * j + h], sh)) << (4 * h);
     o[j] = d;
   }
   st16(codes + (long long)r * (K_pad / 2) + b * 16, o);

@@ -15,8 +15,7 @@ template <int FMT>
 struct MxSpec;
 template <>
 struct MxSpec<MX_E4M3> {
-  static constexpr int MB = 3, EB = 4, BIAS = 7, EMIN = -6, EMAX = 8, BPL = 32, HW = 0;
-  static constexpr float VMAX = 448.0f;
+  static constexpr int EMAX = 8, BPL = 32, HW = 0;
 };
 template <>
 struct MxSpec<MX_E2M1> {
@@ -32,10 +31,9 @@ MKD_DEV int floor_log2_pos(float a) {
   return (31 - __clz(b & 0x7fffffu)) - 149;
 }
 
-// Element code of v (already divided by the block scale): RNE, saturating.
-template <int FMT>
-MKD_DEV uint32_t mx_encode(float v) {
-  using S = MxSpec<FMT>;
+// E2M1 code of v (already divided by the block scale): RNE, saturating (NaN: 6).
+MKD_DEV uint32_t mx_encode_e2m1(float v) {
+  using S = MxSpec<MX_E2M1>;
   const uint32_t sign = __float_as_uint(v) >> 31;
   const float a = fabsf(v);
   const int e = a > 0.f ? max(floor_log2_pos(a), S::EMIN) : S::EMIN;
@@ -55,8 +53,8 @@ MKD_DEV uint32_t mx_encode(float v) {
 
 // Four E4M3 codes (v[0] lowest byte) by gfx950's v_cvt_pk_fp8_f32: round to nearest
 // even, subnormals included; the magnitude is clamped to 448 first, so nothing
-// overflows and a NaN becomes +-448 -- mx_encode<MX_E4M3>'s codes for every fp32
-// pattern, at ~3 instructions per value instead of ~25.
+// overflows and a NaN becomes +-448 (every code, tie and neighbour of a tie against
+// the oracle: tests/test_gpu_mx.py).  ~3 instructions per value, ~25 in integer math.
 MKD_DEV float mx_clamp448(float v) { return __builtin_copysignf(fminf(fabsf(v), 448.0f), v); }
 MKD_DEV uint32_t mx_encode4_e4m3(float a, float b, float c, float d) {
   int o = __builtin_amdgcn_cvt_pk_fp8_f32(mx_clamp448(a), mx_clamp448(b), 0, false);

@@ -50,6 +50,42 @@ def test_quantize_mx_bit_exact(mk, dev, rows, K, dtype, fmt):
     np.testing.assert_array_equal(codes.cpu().numpy(), want_c)
 
 
+def test_quantize_e4m3_every_code_and_tie(mk, dev):
+    """E4M3 codes of every magnitude, of the ties between neighbours and of the floats beside a tie (fp32)
+    and of the ties alone (bf16), subnormals, saturation above 448 and signed zeros included, equal the
+    oracle's; a NaN becomes +-448 and an infinity +-448 under the largest scale."""
+    from nki_moe_megakernel_amd import mx
+    mags = omx.decode_elements(np.arange(127), "e4m3").astype(np.float32)       # 0 .. 448
+    ties = (mags[:-1] + mags[1:]) / 2
+    more = np.array([449.0, 463.9, 464.0, 464.1, 480.0, 511.0], np.float32)     # all code 0x7e
+    near = [np.nextafter(ties, np.float32(0)), np.nextafter(ties, np.float32(1000)), more]
+    for dtype, vals in ((torch.float32, np.concatenate([mags, ties, *near])),
+                        (torch.bfloat16, np.concatenate([mags, ties]))):
+        vals = np.concatenate([vals, -vals])
+        x = np.zeros((-(-len(vals) // 31), 32), np.float32)
+        x[:, 0] = 448.0                                                         # every block's scale is 1
+        body = np.zeros(x.shape[0] * 31, np.float32)
+        body[:len(vals)] = vals
+        x[:, 1:] = body.reshape(-1, 31)
+        xt = torch.from_numpy(x).to(dtype)
+        assert torch.equal(xt.float(), torch.from_numpy(x))
+        codes, scales = mx.quantize_mx(xt.to(dev), FMT["e4m3"], 128)
+        oc, os_ = omx.quantize_mx(x, "e4m3")
+        assert (os_ == 127).all()
+        np.testing.assert_array_equal(codes.cpu().numpy()[:, :32], oc)
+        np.testing.assert_array_equal(scales.cpu().numpy()[:, :1], os_)
+    x = torch.ones(3, 32)
+    x[0, 3], x[0, 5] = float("nan"), -float("nan")
+    x[1, 3], x[1, 5] = float("inf"), -2.0
+    x[2, 3], x[2, 5] = -float("inf"), 2.0
+    codes, scales = (t.cpu().numpy() for t in mx.quantize_mx(x.to(dev), FMT["e4m3"], 128))
+    # amax 1: scale 2^-8, 1 -> 256 (0x78); with an infinity 2^(128 - 8), finite values -> +-0
+    assert scales[:, 0].tolist() == [127 - 8, 247, 247]
+    assert (codes[0, 3] & 0x7f) == 0x7e and (codes[0, 5] & 0x7f) == 0x7e and codes[0, 4] == 0x78
+    assert codes[1, 3] == 0x7e and codes[1, 5] == 0x80 and codes[1, 4] == 0
+    assert codes[2, 3] == 0xfe and codes[2, 5] == 0 and codes[2, 4] == 0
+
+
 def reference_gate_up_layout(codes_l, scales_l, I, fmt):
     """Logical [E, 2I, H] codes (one per element) + [E, 2I, H/32] scales -> the
     reference [E, 128, 2, H/512, I, x4] codes and [E, 16, 2, H/512, I] scales:
