@@ -92,12 +92,14 @@ def test_moe_prefill_rejects_unsupported(mk, dev):
 
 
 # Group sizes at the edges of the token tiles (160, and the equal parts of larger
-# groups) and of the inner loops (32 .. 160 tokens), and k steps (H / 32, I / 32) that leave the four-step loop
-# after any step.  Same tolerance as above: bf16 h and fp32 sums over K <= 416.
-@pytest.mark.parametrize("H,I", [(32, 32), (64, 96), (96, 160), (128, 224), (288, 64), (416, 128)])
+# groups, 200 and 210 in two of 100 .. 112) and of the inner loops (32 .. 160 tokens), and k steps (H / 32,
+# I / 32) that leave the four-step loop after any step, or fill it several times over so that every slot of
+# the token ring is reused (512, 384: 16 and 12 steps of the loops for whole groups of four).  Same tolerance
+# as above: bf16 h and fp32 sums over K <= 512.
+@pytest.mark.parametrize("H,I", [(32, 32), (64, 96), (96, 160), (128, 224), (288, 64), (416, 128), (512, 384)])
 def test_moe_prefill_group_and_k_edges(mk, dev, H, I):
     from nki_moe_megakernel_amd.common_types import ExpertAffinityScaleMode
-    counts = [0, 1, 31, 32, 33, 64, 65, 96, 97, 112, 113, 127, 128, 129, 144, 145, 160, 161, 321, 0]
+    counts = [0, 1, 31, 32, 33, 64, 65, 96, 97, 112, 113, 127, 128, 129, 144, 145, 160, 161, 321, 200, 210, 0]
     print(f"moe_prefill group edges H={H} I={I}", flush=True)
     E, T = len(counts), sum(counts)
     x, gu, dn, _, _, _, _ = _case(T, E, 1, H, I, False, seed=H + I)
