@@ -223,9 +223,10 @@ MKD_DEV void tile_body(const GemmArgs& a, const TileJob& jb, char* lds) {
     mul(f1, b1, H0);
     load_a(f1, 2 * s + 1 + AD);
   };
-  // PAIRS (S a multiple of 4, every shape of the two models): one exit, so that the
-  // compiler's counts at the loop head are those of a full turn.  Otherwise the
-  // loop leaves after any step; the early exits cost it deeper waits.
+  // PAIRS (S a multiple of 4: 2048, 768 and the padded 3072 of the two models): one exit,
+  // so that the compiler's counts at the loop head are those of a full turn.  Otherwise
+  // (2880 is 90 steps) the loop leaves after any step; the early exits cost it deeper
+  // waits, and there is one form, for 160 tokens, whatever the tile holds.
   if (PAIRS) {
     for (int s = 0; s < NS; s += 2) {
       first(s, af[0]);
@@ -311,9 +312,9 @@ MKD_DEV void tile_body(const GemmArgs& a, const TileJob& jb, char* lds) {
     // Each wave turns its 64 rows x 16 tokens through its own 4 KiB of LDS and stores
     // 256 contiguous bytes per token (16 lanes x 16 bytes), with no barrier among
     // the waves.  Straight from the registers a store covers 64 bytes of each of 16
-    // rows: 2048 tokens 119 instead of 112 us.  The grouped rows (T K of them) are
-    // read back once, by the finalize: non-temporal, 2.7 % of moe_prefill at 8192
-    // tokens; the dense rows are the next kernel's input.
+    // rows: 2048 tokens 119 instead of 112 us.  (Non-temporal stores of the grouped rows
+    // make no difference: moe_prefill at 1003 tokens 274.6 us plain and 274.9, at 8192
+    // 794.2 and 794.3.)
     constexpr int kLd = 68;                           // 64 rows + 4 floats of padding
     float* stg = reinterpret_cast<float*>(lds) + w * 16 * kLd;
     __syncthreads();                                  // every wave is past its last operand reads
@@ -350,8 +351,7 @@ MKD_DEV void tile_body(const GemmArgs& a, const TileJob& jb, char* lds) {
         for (int e = 0; e < 4; ++e) v[e] = (v[e] + bb[e]) * sc;
         float* y = ybase + (long long)row * a.ldy + n;
         if (n + 3 < a.N) {
-          if (a.grp_expert) __builtin_nontemporal_store(v, reinterpret_cast<f32x4_t*>(y));
-          else *reinterpret_cast<f32x4_t*>(y) = v;
+          *reinterpret_cast<f32x4_t*>(y) = v;
         } else {
 #pragma unroll
           for (int e = 0; e < 4; ++e)
