@@ -15,8 +15,11 @@
 // block-table round trip per chunk instead of one per tile pair.  At 64 sequences
 // of 512 .. 8192 positions on a paged cache the former form (256-position chunks,
 // each wave loading K, then V, of two tiles at a time, every lane dividing for its
-// own table entry) took 161 us per layer, this one 111 (5.1 TB/s); FP8 at 16 x 4096
-// positions 300 us in plain VALU math (attn_kvfmt_kernel), 29 here.
+// own table entry) took 161 us per layer, this one 108-111 (554 MB fetched, 5.1 TB/s);
+// FP8 at 16 x 4096 positions 300 us in plain VALU math (attn_kvfmt_kernel), 29 here
+// (72 MB fetched, 50 of them rows: the mask's lines are read by every XCD).  The masked
+// bf16 forms of 128-wide heads spill 11 to 13 registers (the eight mask bytes a lane
+// holds a step ahead); no other form does.
 //
 // FP8 caches (e4m3 codes, attention_block_tkg.py:133-134, :749-754): a code is
 // exactly a bf16 value, so the scores are those of the stored values with fp32
@@ -411,10 +414,13 @@ __global__ void __launch_bounds__(64 * kStWaves, FP8 && D == 64 ? 4 : 3) attn_st
 
 namespace {
 
-// Non-temporal loads where the cache cannot be in the 256 MB memory-side cache at
-// the next step (here: its capacity is at least twice that): 64 sequences x 8192,
-// flat 113 -> 103 us, paged 122 -> 111 with the chunk-first order; at 16 x 8192 (146 MB
-// attended) they cost a re-run of the same layer 30 -> 37 us.
+// Non-temporal loads where one layer's cache is at least twice the 256 MB memory-side
+// cache.  Whole steps of 6 layers, always / this rule / never: 64 sequences x 8128
+// 2.29-2.40 / 2.29-2.38 / 2.45 ms, 32 x 8128 1.79-1.81 / 1.80-1.81 / 1.86 ms.  Smaller
+// caches gain too within a model, where the other layers' caches lie between two uses
+// (64 x 2048 1.81-1.84 / 1.82-1.86 / 1.84-1.85 ms; 64-wide heads, 32 x 4096, 4 layers,
+// 1001 / 1009 us); the line is where it is for a layer called again and again on one
+// cache (16 x 8128: 231 / 223 / 224 us).
 template <int D, int GQA>
 hipError_t stream_launch(const AttnArgs& a, hipStream_t s) {
   const dim3 grid(a.nkv, a.n_chunks, a.B), block(64 * kStWaves);
