@@ -40,7 +40,8 @@ def attention_block_tkg(
     generalisation); attention_mask [S_ctx, B, q_heads, S_tkg] with the active
     token in slot S_ctx - 1; kv_cache_update_idx [B, 1] (uint32 max = skip);
     W_out [q_heads*d, H].  out is [B*S_tkg, H] (or [B, q_heads, d, S_tkg]
-    without W_out).  The caches are updated in place.
+    without W_out).  The caches are updated in place.  X_hidden_dim_actual is not
+    used: the input norm's mean runs over all H columns, zero padding included.
 
     Block (paged) KV cache (attention_block_tkg.py:199-206, 699-707,
     1473-1685): with active_blocks_table [B, num_active_blocks], K_cache /
